@@ -10,12 +10,12 @@
 
 namespace skv {
 
-constexpr int DN_WAVES = 8;                // waves per dense block
+constexpr int DN_WAVES = 12;               // waves per dense block
 constexpr int DN_BLOCK = DN_WAVES * 64;
 constexpr int DN_TILE = 16;                // keys per wave iteration (one MFMA row block)
 constexpr int DN_TARGET_BLOCKS = 64;       // partials per KV group (upper bound): one block per CU
-constexpr int DN_MERGE_SLICES = 32;        // 8-dim output slices per query head in the merge
-constexpr int DN_PAGED_MAX_TILES = 128;    // tiles per wave whose record index a paged wave holds
+constexpr int DN_MERGE_SLICES = 8;         // 32-dim output slices per query head in the merge
+constexpr int DN_PAGED_MAX_PAIRS = 64;     // pairs per wave whose record indices a paged wave holds
 
 struct DenseArgs {
   const uint8_t* kv8;   // [G][rows][512]: fp8 V | fp8 K; paged: the page pool
@@ -25,19 +25,29 @@ struct DenseArgs {
   const uint16_t* q;    // [16][256] bf16
   int T;                // keys attended (rows 0 .. T-1 of each group)
   int rows;             // records per group in kv8
-  int iters;            // 16-key tiles per wave
   int nb;               // blocks (partials) per KV group
-  float* part;          // [G][nb][H][D + 2]: unnormalised o, max (log2 units), sum
+  int share, extra;     // pairs of tiles per block (dense_split)
+  float* part;          // [G][nb][H][D] unnormalised o, then [G][nb][H] (max, sum) pairs;
+                        // 16-byte aligned
   uint16_t* out;        // [16][256] bf16
 };
 
-// 16-key tiles per wave and blocks per group for a context of T keys.
-inline void dense_shape(int T, int& iters, int& nb) {
-  const int tiles = (T + DN_TILE - 1) / DN_TILE;
-  iters = (tiles + DN_TARGET_BLOCKS * DN_WAVES - 1) / (DN_TARGET_BLOCKS * DN_WAVES);
-  if (iters < 1) iters = 1;
-  nb = (tiles + iters * DN_WAVES - 1) / (iters * DN_WAVES);
-  if (nb < 1) nb = 1;
+// Blocks (partials) per KV group for a context of T keys, and the pairs of
+// tiles of each: share, one more for the first `extra` blocks.  One pair per
+// block until every CU has a block, so that a short context's records are
+// read by as many CUs as it has pairs.
+inline void dense_split(int T, int& nb, int& share, int& extra) {
+  const int pairs = (T + 2 * DN_TILE - 1) / (2 * DN_TILE);
+  nb = pairs < 1 ? 1 : pairs < DN_TARGET_BLOCKS ? pairs : DN_TARGET_BLOCKS;
+  share = pairs / nb;
+  extra = pairs % nb;
+}
+
+// Most pairs a wave of a block takes.
+inline int dense_wave_pairs(int T) {
+  int nb, share, extra;
+  dense_split(T, nb, share, extra);
+  return (share + (extra ? 1 : 0) + DN_WAVES - 1) / DN_WAVES;
 }
 
 // k = 0: the per-block partials; k = 1: the merge into the output.

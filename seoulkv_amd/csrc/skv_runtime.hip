@@ -516,21 +516,17 @@ static int create_impl(const skv_index_desc* ix, const uint16_t* k_bf16, const u
   const int max_slices = (a.sink + a.local + cap_app + DENSE_SLICE_KEYS - 1) / DENSE_SLICE_KEYS;
   h->dn.T = T;
   h->dn.rows = T + cap_app;
-  dense_shape(T, h->dn.iters, h->dn.nb);
+  dense_split(T, h->dn.nb, h->dn.share, h->dn.extra);
   if (h->dn.nb > DN_TARGET_BLOCKS) {  // the merge kernel holds at most this many partials
     fail(h, SKV_EINVAL, "dense decode shape: %d blocks per group", h->dn.nb);
     return bail(SKV_EINVAL);
   }
-  {  // the paged dense kernel holds the record index of each wave's tiles in
-     // two registers: at most DN_PAGED_MAX_TILES tiles per wave at the largest
-     // context the handle can reach
-    int it = 0, nb = 0;
-    dense_shape(T + cap_app, it, nb);
-    if (pages && it > DN_PAGED_MAX_TILES) {
-      fail(h, SKV_EINVAL, "paged dense decode: %d tiles per wave (at most %d)", it,
-           DN_PAGED_MAX_TILES);
-      return bail(SKV_EINVAL);
-    }
+  // the paged dense kernel holds the record indices of a wave's pairs in its
+  // lanes: at most DN_PAGED_MAX_PAIRS at the largest context the handle can reach
+  if (pages && dense_wave_pairs(T + cap_app) > DN_PAGED_MAX_PAIRS) {
+    fail(h, SKV_EINVAL, "paged dense decode: %d key pairs per wave (at most %d)",
+         dense_wave_pairs(T + cap_app), DN_PAGED_MAX_PAIRS);
+    return bail(SKV_EINVAL);
   }
 
   // ---- static arena
@@ -1069,7 +1065,7 @@ static int append_tokens(Handle* h, const uint16_t* k, const uint16_t* v, int n,
   a.local += n;
   a.dense_slices = (a.sink + a.local + DENSE_SLICE_KEYS - 1) / DENSE_SLICE_KEYS;
   h->dn.T = a.T;
-  dense_shape(a.T, h->dn.iters, h->dn.nb);
+  dense_split(a.T, h->dn.nb, h->dn.share, h->dn.extra);
   drop_graph(h);  // the step's launch shapes changed
   build_meta(h);
   return SKV_OK;

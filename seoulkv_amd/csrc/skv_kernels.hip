@@ -1343,12 +1343,19 @@ __device__ __forceinline__ void load_code4(const uint8_t* rec, int kb, uint32_t 
 // 8-bit dot is 16 x (the 4-bit code dot) + (the residual-4 dot), so one pass
 // over a key's record gives both; the top-256 ranks the 4-bit scores and the
 // top-100 the 8-bit scores of the top-256 union (U2), read from this list by
-// U1 position.  Block b of a group owns a contiguous span of bitmap words:
-// it counts the members in all earlier words (its output base), lists its
-// own members in LDS, copies their tokens to the output list and scores
-// them 16 keys per MFMA tile.  64 blocks of 1024 threads per group, one per
-// CU across the 4 groups, each listing up to 16 words per pass (config 2:
-// one pass).
+// U1 position.  Block b of a group owns an even share of the bitmap words,
+// however few there are: it counts the members in all earlier words (its
+// output base), lists its own members in LDS, copies their tokens to the
+// output list and scores them 16 keys per MFMA tile.  64 blocks of 1024
+// threads per group, one per CU across the 4 groups.
+//
+// Bound by a chain of dependent reads (pool size -> bitmap words -> records),
+// so the work between them is kept short: wave j takes word j of a pass (its
+// lanes are the word's 64 keys), a lane's place in the list is its rank in
+// the word plus the sums of two 16-entry LDS rows, and one barrier lies
+// between the words and the list, one between the list and the records.
+// (Shares of at least 16 words left a pool of 6000 keys to 6 blocks, 9.8 us;
+// words listed through LDS took five barriers.)
 constexpr int US_BLOCK = 1024;
 constexpr int US_GRID = 64;  // blocks per group over the pool
 
@@ -1360,12 +1367,14 @@ __global__ __launch_bounds__(US_BLOCK) void k_union_score(const int* count_word,
                                                           const uint64_t* bm_in,
                                                           const int* tok_base, int W,
                                                           int tok_stride, StepArgs a) {
-  constexpr int US_CHUNK = US_BLOCK / 64;  // bitmap words listed per pass (1 item per thread)
+  constexpr int US_CHUNK = US_BLOCK / WAVE;  // bitmap words per pass: one per wave
+  static_assert(US_CHUNK == 16, "block sums read 16 entries with one row of lanes");
   SKV_TSB(3, 0);
   const int ts = 8;
   SKV_TS(ts, 0);
   const int g = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n_in = count_word[g * ST_WORDS];
   const int words_in = (n_in + 63) / 64;
   const uint64_t* __restrict__ bm = bm_in + (size_t)g * H * W;
@@ -1383,7 +1392,7 @@ __global__ __launch_bounds__(US_BLOCK) void k_union_score(const int* count_word,
     SKV_TSE(3);
     return;
   }
-  const int span = max(US_CHUNK, (words_in + (int)gridDim.x - 1) / (int)gridDim.x);
+  const int span = (words_in + (int)gridDim.x - 1) / (int)gridDim.x;
   const int w_lo = blockIdx.x * span;
   if (w_lo >= words_in) {
     SKV_TSE(3);
@@ -1391,19 +1400,14 @@ __global__ __launch_bounds__(US_BLOCK) void k_union_score(const int* count_word,
   }
   const int w_hi = min(words_in, w_lo + span);
 
-  __shared__ int s_red[US_BLOCK / WAVE + 1];
-  __shared__ uint64_t s_word[US_CHUNK];
-  __shared__ int s_wbase[US_CHUNK + 1];
+  __shared__ int s_red[US_CHUNK], s_cnt[US_CHUNK];
   __shared__ int s_tok[US_CHUNK * 64];
   auto word = [&](int w) { return bm[w] | bm[W + w] | bm[2 * W + w] | bm[3 * W + w]; };
 
-  // issued together: the member counts of words [0, w_lo) (4 words, 16
-  // loads in flight per thread), the first chunk's words (one bitmap word per
-  // thread < 4 US_CHUNK) and its input tokens (one per thread)
-  const int nw0 = min(US_CHUNK, w_hi - w_lo);
-  uint64_t hw = 0;
-  if ((int)threadIdx.x < H * nw0) hw = bm[(threadIdx.x / nw0) * W + w_lo + threadIdx.x % nw0];
-  const int tok0 = (int)threadIdx.x < 64 * nw0 ? tok_in[64 * w_lo + threadIdx.x] : 0;
+  // issued together: this wave's word and its 64 keys' tokens, and the member
+  // counts of words [0, w_lo) (4 words, 16 loads in flight per thread)
+  uint64_t mine = w_lo + wave < w_hi ? word(w_lo + wave) : 0ull;
+  int tok = w_lo + wave < w_hi ? tok_in[64 * (w_lo + wave) + lane] : 0;
   int cnt = 0;
   for (int w = threadIdx.x; w < w_lo; w += 4 * US_BLOCK) {
     uint64_t m[4];
@@ -1415,16 +1419,6 @@ __global__ __launch_bounds__(US_BLOCK) void k_union_score(const int* count_word,
 #pragma unroll
     for (int u = 0; u < 4; ++u) cnt += __popcll(m[u]);
   }
-  if (threadIdx.x < US_CHUNK) s_word[threadIdx.x] = 0;
-  cnt = wave_sum(cnt);
-  if (lane == 0) s_red[wave] = cnt;
-  __syncthreads();
-  if (hw) atomicOr(reinterpret_cast<unsigned long long*>(&s_word[threadIdx.x % nw0]), hw);
-  int base = 0;
-#pragma unroll
-  for (int i = 0; i < US_BLOCK / WAVE; ++i) base += s_red[i];
-  SKV_TS(ts, 1);
-
   const QOperand* q = &a.qop[g * QV_COUNT + QV_QS];
   uint32_t b[4][4];
   load_b(q, b);
@@ -1432,47 +1426,45 @@ __global__ __launch_bounds__(US_BLOCK) void k_union_score(const int* count_word,
   // lane l converts key l % 16 of a tile for head l / 16:
   // 4-bit (2 dq - 15 S) 2^(fx + 4), 8-bit (2 dq - 255 S) 2^fx
   const int hq = lane >> 4;
-  const LimbScale ls4(q->fx[hq] + 4, 1), ls8(q->fx[hq], 1);
-  const double lc4 = LimbScale::offset(-15 * q->sum[hq], q->fx[hq] + 4);
-  const double lc8 = LimbScale::offset(-255 * q->sum[hq], q->fx[hq]);
+  const int fx = q->fx[hq];
+  const int64_t sum = q->sum[hq];
+  cnt = wave_sum(cnt);
+  if (lane == 0) s_red[wave] = cnt;
+  const LimbScale ls4(fx + 4, 1), ls8(fx, 1);
+  const double lc4 = LimbScale::offset(-15 * sum, fx + 4);
+  const double lc8 = LimbScale::offset(-255 * sum, fx);
+  int base = 0;  // output base of the pass (read with its first counts)
   for (int c0 = w_lo; c0 < w_hi; c0 += US_CHUNK) {
-    const int nw = min(US_CHUNK, w_hi - c0);
-    const bool first = c0 == w_lo;
-    if (!first) {  // later chunks (long inputs): the union words now
-      __syncthreads();
-      if (threadIdx.x < US_CHUNK) s_word[threadIdx.x] = (int)threadIdx.x < nw ? word(c0 + threadIdx.x) : 0ull;
+    if (c0 != w_lo) {  // later passes (long inputs): the word and its tokens now
+      const int w = c0 + wave;
+      mine = w < w_hi ? word(w) : 0ull;
+      tok = w < w_hi ? tok_in[64 * w + lane] : 0;
+      __syncthreads();  // the previous pass's list has been read
     }
+    if (lane == 0) s_cnt[wave] = __popcll(mine);
     __syncthreads();
-    if (threadIdx.x < 64) {  // wave 0: the member base of each word
-      const uint64_t m = lane < US_CHUNK ? s_word[lane] : 0ull;
-      const int pc = __popcll(m);
-      const int inc = wave_incl_scan(pc);
-      if (lane < US_CHUNK) s_wbase[lane] = inc - pc;
-      if (lane == US_CHUNK - 1) s_wbase[US_CHUNK] = inc;
-    }
-    __syncthreads();
-    const int nloc = s_wbase[US_CHUNK];
-    // list the chunk's members: thread t tests bit t % 64 of word t / 64
-    {
-      const int j = threadIdx.x >> 6, bit = threadIdx.x & 63;
-      const uint64_t m = s_word[j];
-      if ((m >> bit) & 1ull) {
-        const int r = s_wbase[j] + __popcll(m & ((1ull << bit) - 1));
-        const int t = first ? tok0 : tok_in[64 * (c0 + j) + bit];
-        s_tok[r] = t;
-        if (base + r < U1_MAX) tok_out[base + r] = t;
-      }
+    SKV_TS(ts, 1);
+    // members of the earlier waves' words, of the pass, and (first pass) of
+    // all earlier words: one row of 16 lanes each
+    const int inc = wave_incl_scan(lane < US_CHUNK ? s_cnt[lane] : 0);
+    const int nloc = __builtin_amdgcn_readlane(inc, US_CHUNK - 1);
+    const int before = wave ? __builtin_amdgcn_readlane(inc, wave - 1) : 0;
+    if (c0 == w_lo) base = wave_sum(lane < US_CHUNK ? s_red[lane] : 0);
+    if ((mine >> lane) & 1ull) {
+      const int r = before + __popcll(mine & ((1ull << lane) - 1ull));
+      s_tok[r] = tok;
+      if (base + r < U1_MAX) tok_out[base + r] = tok;
     }
     __syncthreads();
     // scores of the listed members, one 16-key tile per wave at a time
-    for (int tile = wave; tile * 16 < nloc; tile += US_BLOCK / WAVE) {
+    for (int tile = wave; tile * 16 < nloc; tile += US_CHUNK) {
       const int i_in = tile * 16 + row;
       uint32_t hi[4][4] = {}, lo[4][4] = {};
       if (i_in < nloc) {
         const uint8_t* rec = a.keyrec + ((size_t)g * a.rec_rows + s_tok[i_in]) * 256;
-        load_code4(rec, kb, hi);
         const uint4 r0 = *reinterpret_cast<const uint4*>(rec + 128 + kb * 32);
         const uint4 r1 = *reinterpret_cast<const uint4*>(rec + 128 + kb * 32 + 16);
+        load_code4(rec, kb, hi);
         const uint32_t rw[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
 #pragma unroll
         for (int kc = 0; kc < 4; ++kc) expand4t(rw[2 * kc], rw[2 * kc + 1], lo[kc]);
@@ -1494,7 +1486,6 @@ __global__ __launch_bounds__(US_BLOCK) void k_union_score(const int* count_word,
       }
     }
     base += nloc;
-    __syncthreads();
   }
   if (w_hi == words_in && threadIdx.x == 0) a.status[g * ST_WORDS + ST_U1] = min(base, U1_MAX);
   SKV_TS(ts, 15);

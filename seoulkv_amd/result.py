@@ -18,9 +18,13 @@ import torch
 
 
 class _DeviceArray:
-    """__cuda_array_interface__ wrapper of a raw device pointer."""
+    """__cuda_array_interface__ wrapper of a raw device pointer.  ``owner``
+    (whose memory it is) lives as long as the wrapper, which PyTorch keeps for
+    as long as a tensor over it: a view outlives the instance it was taken
+    from being dropped (not its ``close()``)."""
 
-    def __init__(self, ptr: int, shape, typestr: str):
+    def __init__(self, ptr: int, shape, typestr: str, owner):
+        self.owner = owner
         self.__cuda_array_interface__ = {
             "shape": tuple(shape),
             "typestr": typestr,
@@ -54,7 +58,7 @@ class DecodeResult:
         state = owner._require_initialized()
         ptr = state.output_tiles_device_ptr()
         raw = torch.as_tensor(
-            _DeviceArray(ptr, (4, 1, 32, 4, 256), "<i2"), device=f"cuda:{owner._device}"
+            _DeviceArray(ptr, (4, 1, 32, 4, 256), "<i2", state), device=f"cuda:{owner._device}"
         ).view(torch.bfloat16)
         return tuple(raw[g] for g in range(4))
 

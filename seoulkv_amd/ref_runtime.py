@@ -60,7 +60,8 @@ class GroupOutput:
         from seoulkv_amd.result import _DeviceArray
 
         raw = torch.as_tensor(
-            _DeviceArray(self._runtime.output_tiles_device_ptr(), (4,) + self.shape, "<i2"),
+            _DeviceArray(self._runtime.output_tiles_device_ptr(), (4,) + self.shape, "<i2",
+                         self._runtime),
             device=f"cuda:{self._runtime.device}",
         ).view(torch.bfloat16)
         return raw[self.slot]

@@ -23,7 +23,7 @@ class _DeviceArray:
     as long as a tensor over it: a view outlives the instance it was taken
     from being dropped (not its ``close()``)."""
 
-    def __init__(self, ptr: int, shape, typestr: str, owner):
+    def __init__(self, ptr: int, shape, typestr: str, owner=None):
         self.owner = owner
         self.__cuda_array_interface__ = {
             "shape": tuple(shape),

@@ -232,31 +232,37 @@ __device__ __forceinline__ unsigned wave_incl_scan_u(unsigned v) {
   return v;
 }
 
-// Exclusive block scan of one value per thread; returns the exclusive prefix
-// and stores the block total in *total.  scratch: >= blockDim/64 + 1 words.
-// T = int, or unsigned for packed fields whose sums may pass 2^31.
+// Inclusive scan within each row of 16 lanes.
+__device__ __forceinline__ int row_incl_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);  // row_shr:8
+  return v;
+}
+
+constexpr int SCAN_WAVES = 16;  // blocks that scan: 1024 threads, 16 waves
+
+// Exclusive block scan of one value per thread (1024 threads): returns the
+// exclusive prefix and the block total in *total.  scratch: SCAN_WAVES words.
+// T = int, or unsigned for packed fields whose sums may pass 2^31.  One
+// barrier: every wave publishes its total and then scans the 16 of them
+// itself (a second pass by one wave between two more barriers took 0.2 us
+// more).  The block must pass a barrier of the caller's before scratch is
+// written again.
 template <typename T>
 __device__ __forceinline__ T block_excl_scan_t(T v, T* scratch, T* total) {
-  const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-  const int nw = (blockDim.x + WAVE - 1) / WAVE;
-  auto scan = [](T x) -> T {
-    if constexpr (sizeof(T) == 4 && T(-1) > T(0)) return wave_incl_scan_u(x);
-    else return wave_incl_scan(x);
-  };
-  T inc = scan(v);
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  T inc;
+  if constexpr (T(-1) > T(0)) inc = wave_incl_scan_u(v);
+  else inc = wave_incl_scan(v);
   if (lane == WAVE - 1) scratch[wave] = inc;
   __syncthreads();
-  if (wave == 0) {
-    T w = lane < nw ? scratch[lane] : T(0);
-    T winc = scan(w);
-    if (lane < nw) scratch[lane] = winc - w;
-    if (lane == nw - 1) scratch[nw] = winc;
-  }
-  __syncthreads();
-  T res = inc - v + scratch[wave];
-  *total = scratch[nw];
-  __syncthreads();
-  return res;
+  const int winc = row_incl_scan(lane < SCAN_WAVES ? (int)scratch[lane] : 0);
+  *total = (T)__builtin_amdgcn_readlane(winc, SCAN_WAVES - 1);
+  const T before = wave ? (T)__builtin_amdgcn_readlane(winc, wave - 1) : T(0);
+  return before + (inc - v);
 }
 
 __device__ __forceinline__ int block_excl_scan(int v, int* scratch, int* total) {

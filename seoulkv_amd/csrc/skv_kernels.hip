@@ -48,7 +48,7 @@ __device__ unsigned long long g_skv_trace_blk[12][4096][4];
 // variant) and the int8 limb B image, written to *out (LDS or global
 // memory).  Sum of squares: X^2 < 2^44 is split into 22-bit halves so that
 // both wave sums stay below 2^30 (exact in int32).
-__device__ void prep_head(const StepArgs& a, int g, int v, QOperand* out, int h, int lane,
+__device__ __forceinline__ void prep_head(const StepArgs& a, int g, int v, QOperand* out, int h, int lane,
                           uint2 qw, bool own);
 
 // This lane's 4 BF16 query elements of head h of group g (dims 4 lane ..).
@@ -60,7 +60,7 @@ __device__ __forceinline__ uint2 load_qw(const StepArgs& a, int g, int h, int la
 // operand is complete after the barrier.  Later waves repeat head H - 1 and
 // write nothing: every thread uses its query word, so the compiler keeps
 // the caller's query load where the caller issued it (first).
-__device__ void prep_operand(const StepArgs& a, int g, int v, QOperand* out, uint2 qw) {
+__device__ __forceinline__ void prep_operand(const StepArgs& a, int g, int v, QOperand* out, uint2 qw) {
   const int lane = threadIdx.x & 63, h = threadIdx.x >> 6;
   prep_head(a, g, v, out, min(h, H - 1), lane, qw, h < H);
   __syncthreads();
@@ -68,7 +68,7 @@ __device__ void prep_operand(const StepArgs& a, int g, int v, QOperand* out, uin
 
 // One wave per head: the integers X, their sum, the scale exponent and
 // ||q|| lambda (raw variant) of query head 4g + h.
-__device__ void prep_head(const StepArgs& a, int g, int v, QOperand* out, int h, int lane,
+__device__ __forceinline__ void prep_head(const StepArgs& a, int g, int v, QOperand* out, int h, int lane,
                           uint2 qw, bool own) {
   const uint32_t qb[4] = {qw.x & 0xffffu, qw.x >> 16, qw.y & 0xffffu, qw.y >> 16};
   uint32_t bits[4];
@@ -283,7 +283,7 @@ __device__ __forceinline__ int kv_lane_row(const StepArgs& a, int g, int tk) {
 
 // Dense slice r of query head j: keys r*256 .. r*256+255 of [sink | local].
 template <bool PAGED>
-__device__ void dense_attend(const StepArgs& a, int blk, AttnScratch& s) {
+__device__ __forceinline__ void dense_attend(const StepArgs& a, int blk, AttnScratch& s) {
   const int j = blk / a.dense_slices, r = blk % a.dense_slices, g = j / H;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ndense = a.sink + a.local;
@@ -524,7 +524,7 @@ __device__ __forceinline__ void load_lds_masked(uint16_t* so, const uint16_t* __
 
 // Both selections of one (group, head) with its nc <= OCT_ITEMS centroids
 // held in registers, one octet of lower, upper and fine scores per thread.
-__device__ void select_in_registers(const StepArgs& a, const uint16_t* lower,
+__device__ __forceinline__ void select_in_registers(const StepArgs& a, const uint16_t* lower,
                                     const uint16_t* upper, const uint16_t* fine, int nc, int g,
                                     int h, FastScratch& fs) {
   const int t = threadIdx.x;
@@ -532,14 +532,19 @@ __device__ void select_in_registers(const StepArgs& a, const uint16_t* lower,
   const uint4 wl = load_oct(lower + row, nc);
   const uint4 wu = load_oct(upper + row, nc);
   const uint4 wf = load_oct(fine + row, nc);
-  auto cid = [](int i) { return (uint32_t)i; };
-  const OctResult r1 = oct_select<true, true>(wl, a.P[g], cid, fs, 2);
+  auto cid = [](int) { return 0u; };  // (ties by position)
+  // both selections' histograms, cleared while the rows arrive
+  fs_clear(fs.hist, fs.w[0]);
+  fs_clear(fs.hist_b, fs.w[1]);
+  __syncthreads();
+  const uint4 l1[1] = {wl};
+  const OctResult r1 = octn_select<1, TIE_VALUE>(l1, a.P[g], cid, fs.hist, fs.w[0], fs, 2);
   const uint32_t thr = r1.sel.all ? 0u : r1.sel.v;
   if (t == 0) a.thr[g * H + h] = thr;
   SKV_TS(2, 6);
   // fine scores of the eligible centroids (upper >= thr), others excluded
-  const uint4 wm = MaskedScores::pick4(wf, wu, thr);
-  const OctResult r2 = oct_select<false, true>(wm, a.P[g], cid, fs, 4);
+  const uint4 wm[1] = {MaskedScores::pick4(wf, wu, thr)};
+  const OctResult r2 = octn_select<1, TIE_POS>(wm, a.P[g], cid, fs.hist_b, fs.w[1], fs, 4);
   // items 8t .. 8t+7 are byte t & 3 of bitmap word t >> 2: merge 4 lanes
   uint32_t m = r2.mine << (8 * (t & 3));
   m |= __shfl_xor(m, 1);
@@ -573,8 +578,11 @@ __device__ __forceinline__ bool select_in_registers_n(const StepArgs& a, const u
     wu[o] = load_oct(upper + row + o * OCT_ITEMS, nc - o * OCT_ITEMS);
     wf[o] = load_oct(fine + row + o * OCT_ITEMS, nc - o * OCT_ITEMS);
   }
-  auto cid = [](int i) { return (uint32_t)i; };
-  const OctResult r1 = octn_select<NO, true, false>(wl, a.P[g], cid, fs, 2);
+  auto cid = [t](int b) { return (uint32_t)(8 * (t + (b >> 3) * SEL_BLOCK) + (b & 7)); };
+  fs_clear(fs.hist, fs.w[0]);
+  fs_clear(fs.hist_b, fs.w[1]);
+  __syncthreads();
+  const OctResult r1 = octn_select<NO, TIE_VALUE>(wl, a.P[g], cid, fs.hist, fs.w[0], fs, 2);
   const uint32_t thr = r1.sel.all ? 0u : r1.sel.v;
   if (t == 0) a.thr[g * H + h] = thr;
   *thr_out = thr;
@@ -582,7 +590,7 @@ __device__ __forceinline__ bool select_in_registers_n(const StepArgs& a, const u
   uint4 wm[NO];
 #pragma unroll
   for (int o = 0; o < NO; ++o) wm[o] = MaskedScores::pick4(wf[o], wu[o], thr);
-  const OctResult r2 = octn_select<NO, false, false>(wm, a.P[g], cid, fs, 4);
+  const OctResult r2 = octn_select<NO, TIE_ID>(wm, a.P[g], cid, fs.hist_b, fs.w[1], fs, 4);
   if (!r2.ok) return false;  // block-uniform
   // items 8u .. 8u+7 (u = t + o SEL_BLOCK) are byte u & 3 of bitmap word u >> 2
 #pragma unroll
@@ -642,6 +650,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_select(const uint16_t* lower, con
       // the full selection over the LDS copy of the eligible fine scores
       const size_t row = ((size_t)g * H + h) * nc;
       uint16_t* so = reinterpret_cast<uint16_t*>(dyn);
+      __syncthreads();  // the register selection's scratch has been read
       load_lds_masked(so, fine + row, upper + row, thr, nc);
       __syncthreads();
       const Selection sel = block_select(so, nc, a.P[g], [](int i) { return (uint32_t)i; }, s);
@@ -679,21 +688,21 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_select(const uint16_t* lower, con
     FastScratch& fs = *reinterpret_cast<FastScratch*>(dyn);
     const int nt8 = nc / 8;
     const uint4 wt = load_oct(a.tmax_lo + ((size_t)g * H + h) * nt8, nt8);
-    const OctResult rt = oct_select<true, false>(wt, a.P[g], cid, fs);
+    const OctResult rt = oct_select_clear<TIE_VALUE>(wt, a.P[g], cid, fs);
     const uint32_t x = rt.sel.all ? 1u : rt.sel.v;
     const u32x4 wtv = {wt.x, wt.y, wt.z, wt.w};
     uint32_t fl = 0;
 #pragma unroll
     for (int e = 0; e < 8; ++e) fl |= (uint32_t)(oct_half(wtv, e) >= x) << e;
     int ntiles;
-    int j = block_excl_scan(__popc(fl), fs.scan, &ntiles);  // ends with a barrier
+    int j = block_excl_scan(__popc(fl), fs.w[1].scan, &ntiles);
     if (ntiles <= SEL_BLOCK) {
       int* tl = reinterpret_cast<int*>(fs.cand);
       for (uint32_t rest = fl; rest; rest &= rest - 1) tl[j++] = 8 * (int)threadIdx.x + __ffs(rest) - 1;
       __syncthreads();
       uint4 wg = make_uint4(0, 0, 0, 0);
       if ((int)threadIdx.x < ntiles) wg = reinterpret_cast<const uint4*>(lo)[tl[threadIdx.x]];
-      const OctResult rg = oct_select<true, false>(wg, a.P[g], cid, fs);
+      const OctResult rg = oct_select_clear<TIE_VALUE>(wg, a.P[g], cid, fs);
       if (threadIdx.x == 0) s_thr = rg.sel.all ? 0u : rg.sel.v;
       done = true;
     }
@@ -725,21 +734,23 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_select(const uint16_t* lower, con
   done = false;
   if (a.exact_select != 1) {
     FastScratch& fs = *reinterpret_cast<FastScratch*>(dyn);
-    FastResult r{};
-    r.ok = false;
     if (a.tmax_fi && nc / 16 <= 4 * SEL_BLOCK) {
       // only the 16-centroid tiles whose max fine score reaches the cut can
       // hold a candidate: their scores and gates are loaded, no others
       uint32_t sv[FS_PER];
 #pragma unroll
       for (int u = 0; u < FS_PER; ++u) sv[u] = pg[u] >= thr ? pf[u] : 0u;
-      r = tiled_select(MaskedTiles{fi, up, thr}, a.tmax_fi + ((size_t)g * H + h) * (nc / 16), sv, nc,
-                       a.P[g], cid, fs, force, 4);
+      tiled_clear(fs);
       __syncthreads();
+      done = tiled_select(MaskedTiles{fi, up, thr}, a.tmax_fi + ((size_t)g * H + h) * (nc / 16), sv,
+                          nc, a.P[g], cid, fs, force, 4, [selbm](int tile, uint32_t m) {
+                            atomicOr(&selbm[tile >> 1], m << (16 * (tile & 1)));
+                          });
     }
-    if (!r.ok)
-      r = fast_select_s<false>(MaskedScores{fi, up, thr}, nc, a.P[g], cid, fs, force, 4,
-                               [&](int u, int) { return pg[u] >= thr ? pf[u] : 0u; });
+  }
+  if (!done && a.exact_select != 1) {
+    FastScratch& fs = *reinterpret_cast<FastScratch*>(dyn);
+    const FastResult r = fast_select(MaskedScores{fi, up, thr}, nc, a.P[g], cid, fs, force, 4);
     if (r.ok) {
       for (int c = threadIdx.x; c < r.ncand; c += SEL_BLOCK) {
         const uint64_t key = fs.cand[c];
@@ -912,7 +923,7 @@ __global__ __launch_bounds__(PL_BLOCK) void k_pool(const uint32_t* selbm, const 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = threadIdx.x;
   extern __shared__ uint32_t s_bm[];
   __shared__ int s_off[2 * PL_BLOCK], s_cum[PL_RANGE_MAX + 1], s_cl[PL_RANGE_MAX];
-  __shared__ int s_scan[PL_WAVES + 1], s_surv;
+  __shared__ int s_scan[2][PL_WAVES], s_surv;  // (scans take the two rows in turn)
   __shared__ unsigned long long s_excl;
   __shared__ uint32_t s_tm[H * PL_TM_TILES];  // tile maxima of the first two pages' keys
   // range b = block b: workgroups are dispatched in index order within each
@@ -977,7 +988,7 @@ __global__ __launch_bounds__(PL_BLOCK) void k_pool(const uint32_t* selbm, const 
   const unsigned size = is_sel ? (unsigned)(s_off[t + 1] - s_off[t]) : 0u;
   unsigned tot;
   const unsigned ex = block_excl_scan_t<unsigned>((size << PL_SEL_BITS) | (is_sel ? 1u : 0u),
-                                                  reinterpret_cast<unsigned*>(s_scan), &tot);
+                                                  reinterpret_cast<unsigned*>(s_scan[0]), &tot);
   const int nsel = (int)(tot & PL_SEL_MASK);
   if (is_sel) {
     const int r = (int)(ex & PL_SEL_MASK);
@@ -1031,15 +1042,17 @@ __global__ __launch_bounds__(PL_BLOCK) void k_pool(const uint32_t* selbm, const 
   s2_rows(rows, o1 ? j1 : -1, rw1);
   // one scan for both pages: page 1 in the high half (a page owns < 2^16)
   int both;
-  const int exb = block_excl_scan((o1 ? 1 << 16 : 0) | (o0 ? 1 : 0), s_scan, &both);
+  const int exb = block_excl_scan((o1 ? 1 << 16 : 0) | (o0 ? 1 : 0), s_scan[1], &both);
   const int ex0 = exb & 0xffff, ex1 = exb >> 16;
   const int page0_total = both & 0xffff, page1_total = both >> 16;
   int owned_total = page0_total + page1_total;
+  int flip = 0;
   for (int base = 2 * PL_PAGE; base < S; base += PL_PAGE) {
     int j = 0;
     const bool o = pi >= 0 && base + pi < S && posting(base + pi, j);
     int tot;
-    (void)block_excl_scan(o ? 1 : 0, s_scan, &tot);
+    (void)block_excl_scan(o ? 1 : 0, s_scan[flip], &tot);
+    flip ^= 1;
     owned_total += tot;
   }
   // ---- publish, then look back for the counts of the earlier ranges
@@ -1147,7 +1160,8 @@ __global__ __launch_bounds__(PL_BLOCK) void k_pool(const uint32_t* selbm, const 
     uint4 rw[4];
     if (wave > 0) s2_rows(rows, o ? j : -1, rw);
     int tot;
-    const int ex = block_excl_scan(o ? 1 : 0, s_scan, &tot);
+    const int ex = block_excl_scan(o ? 1 : 0, s_scan[flip], &tot);
+    flip ^= 1;
     const int p = pos0 + carry + ex;
     if (o && p < a.cap) pool[p] = ptok[j];
     uint32_t sc[4] = {0, 0, 0, 0};
@@ -1202,6 +1216,21 @@ size_t topk_dynamic_lds(int lds_items) {
   return std::max(sizeof(FastScratch) + (size_t)TOPK_LDS_WORDS * 8, (size_t)lds_items * 2);
 }
 
+// The 8 token IDs of this thread's octet of a row of n (stride entries, a
+// multiple of 8): tied IDs are then in registers when the tie is known.
+struct TokOct {
+  u32x4 lo, hi;
+  __device__ uint32_t id(int b) const { return b < 4 ? lo[b & 3] : hi[b & 3]; }
+};
+__device__ __forceinline__ TokOct load_tok_oct(const int* __restrict__ tok, int n) {
+  TokOct r = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}};
+  if (8 * (int)threadIdx.x < n) {
+    r.lo = reinterpret_cast<const u32x4*>(tok)[2 * threadIdx.x];
+    r.hi = reinterpret_cast<const u32x4*>(tok)[2 * threadIdx.x + 1];
+  }
+  return r;
+}
+
 // Per (group, head): members = top-k by (ordered score, lowest token) of the
 // n items; writes the membership bitmap.  LDS-resident when n <= lds_items,
 // otherwise 8-bit radix passes over the full 40-bit keys in memory.
@@ -1229,19 +1258,26 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_topk(const int* count_word, const
   const int* tok = t.tokens + (size_t)g * t.stride;
   uint64_t* bm = t.bitmap + ((size_t)g * H + h) * words;
   auto id = [tok](int i) { return (uint32_t)tok[i]; };
-  if (exact_select == 0 && n <= OCT_ITEMS) {  // the scores fit in registers
-    const OctResult r = oct_select<false, false>(load_oct(sc, n), t.k, id,
-                                                 *reinterpret_cast<FastScratch*>(dyn), ts);
+  FastScratch& fs = *reinterpret_cast<FastScratch*>(dyn);
+  if (exact_select == 0 && n <= OCT_ITEMS) {  // the scores fit in registers, and their IDs
+    const uint4 w1[1] = {load_oct(sc, n)};
+    const TokOct tk[1] = {load_tok_oct(tok, n)};
+    fs_clear(fs.hist, fs.w[0]);
+    __syncthreads();
+    const OctResult r = octn_select<1, TIE_ID>(
+        w1, t.k, [&](int b) { return tk[0].id(b); }, fs.hist, fs.w[0], fs, ts);
     if (r.ok) {
       write_member_words(r.mine, n, bm);
       SKV_TS(ts, 15);
       SKV_TSE((t.count_slot == ST_POOL ? 6 : 7));
       return;
     }
+    __syncthreads();  // the scratch is used again below
   } else if (OCT2 && exact_select == 0 && n <= 2 * OCT_ITEMS) {  // two octets per thread
     const uint4 w2[2] = {load_oct(sc, n), load_oct(sc + OCT_ITEMS, n - OCT_ITEMS)};
-    const OctResult r = octn_select<2, false, false>(w2, t.k, id,
-                                                     *reinterpret_cast<FastScratch*>(dyn), ts);
+    fs_clear(fs.hist, fs.w[0]);
+    __syncthreads();
+    const OctResult r = octn_select<2, TIE_LOAD>(w2, t.k, id, fs.hist, fs.w[0], fs, ts);
     if (r.ok) {
       write_member_words(r.mine & 0xffu, OCT_ITEMS, bm);
       write_member_words(r.mine >> 8, n - OCT_ITEMS, bm + OCT_ITEMS / 64);
@@ -1249,29 +1285,38 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_topk(const int* count_word, const
       SKV_TSE((t.count_slot == ST_POOL ? 6 : 7));
       return;
     }
+    __syncthreads();
   }
   if (exact_select != 1) {
-    FastScratch& fs = *reinterpret_cast<FastScratch*>(dyn);
     // the member bitmap: in LDS beside the scratch (cleared before the
     // selection) when it fits, else in place
     const int words = (n + 63) / 64;
     const bool local = words <= TOPK_LDS_WORDS;
     uint64_t* mb = local ? reinterpret_cast<uint64_t*>(dyn + sizeof(FastScratch)) : bm;
-    if (local)
-      for (int w = threadIdx.x; w < words; w += SEL_BLOCK) mb[w] = 0;
-    FastResult r{};
-    r.ok = false;
-    if (tile_max && exact_select != 1 && n > OCT_ITEMS && (n + 15) / 16 <= 4 * SEL_BLOCK) {
+    if (tile_max && n > OCT_ITEMS && (n + 15) / 16 <= 4 * SEL_BLOCK) {
       // the producer wrote the max of every 16-item tile: only the tiles
-      // reaching the cut are read for candidates
+      // reaching the cut are read
+      static_assert(TOPK_LDS_WORDS * 64 >= 64 * SEL_BLOCK, "a tiled row's bitmap is local");
       uint32_t sv[FS_PER];
 #pragma unroll
       for (int u = 0; u < FS_PER; ++u) sv[u] = sc[fs_sample_item(n, u)];
-      r = tiled_select(RowTiles{sc}, tile_max + ((size_t)g * H + h) * t.tile_stride, sv, n, t.k,
-                       id, fs, exact_select == 2, ts);
+      for (int w = threadIdx.x; w < words; w += SEL_BLOCK) mb[w] = 0;
+      tiled_clear(fs);
       __syncthreads();
+      uint16_t* mt = reinterpret_cast<uint16_t*>(mb);  // a tile's members
+      if (tiled_select(RowTiles{sc}, tile_max + ((size_t)g * H + h) * t.tile_stride, sv, n, t.k, id,
+                       fs, exact_select == 2, ts,
+                       [mt](int tile, uint32_t m) { mt[tile] = (uint16_t)m; })) {
+        __syncthreads();
+        for (int w = threadIdx.x; w < words; w += SEL_BLOCK) bm[w] = mb[w];
+        SKV_TS(ts, 15);
+        SKV_TSE((t.count_slot == ST_POOL ? 6 : 7));
+        return;
+      }
     }
-    if (!r.ok) r = fast_select(RowScores{sc}, n, t.k, id, fs, exact_select == 2, ts);
+    if (local)
+      for (int w = threadIdx.x; w < words; w += SEL_BLOCK) mb[w] = 0;
+    const FastResult r = fast_select(RowScores{sc}, n, t.k, id, fs, exact_select == 2, ts);
     if (r.ok) {
       SKV_TS(ts, 6);
       if (!local) {
@@ -1586,38 +1631,30 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
   if (threadIdx.x == 0) s_cnt = 0;
   bool done = false, listed = false;  // listed: s_key is in U2 list order
   if (exact_select == 0) {  // n <= U1_MAX <= OCT_ITEMS: scores and IDs in registers
-    const uint4 w = keep_octet(load_oct(sc, n), ubits);
-    uint4 t0 = make_uint4(0, 0, 0, 0), t1 = t0;
-    if (8 * (int)threadIdx.x < n) {  // rows hold U1_MAX (a multiple of 8) entries
-      t0 = reinterpret_cast<const uint4*>(tok)[2 * threadIdx.x];
-      t1 = reinterpret_cast<const uint4*>(tok)[2 * threadIdx.x + 1];
-    }
-    // the octet's tokens in LDS for the tie ranking (ordered before their
-    // reads by the selection's first barrier)
-    __shared__ __align__(16) uint32_t s_tok[U1_MAX];
-    if (8 * (int)threadIdx.x < U1_MAX) {
-      reinterpret_cast<uint4*>(s_tok)[2 * threadIdx.x] = t0;
-      reinterpret_cast<uint4*>(s_tok)[2 * threadIdx.x + 1] = t1;
-    }
-    const OctResult r = oct_select<false, false>(
-        w, TOPK, [&](int i) { return s_tok[i]; }, *reinterpret_cast<FastScratch*>(dyn), 13);
+    const uint4 w[1] = {keep_octet(load_oct(sc, n), ubits)};
+    const TokOct tk = load_tok_oct(tok, n);  // (rows hold U1_MAX, a multiple of 8, entries)
+    FastScratch& fs = *reinterpret_cast<FastScratch*>(dyn);
+    fs_clear(fs.hist, fs.w[0]);
+    __syncthreads();
+    const OctResult r = octn_select<1, TIE_ID>(
+        w, TOPK, [&](int b) { return tk.id(b); }, fs.hist, fs.w[0], fs, 13);
     if (r.ok) {
       SKV_TS(13, 6);
       // members in list order (deterministic, so the attention sums are too)
       int nm;
       const int base = block_excl_scan(__popc(r.mine), s.scan, &nm);
-      const u32x4 wv = {w.x, w.y, w.z, w.w};
-      const u32x4 ta = {t0.x, t0.y, t0.z, t0.w}, tb = {t1.x, t1.y, t1.z, t1.w};
+      const u32x4 wv = {w[0].x, w[0].y, w[0].z, w[0].w};
       int slot = base;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if (!((r.mine >> e) & 1u)) continue;
-        const uint32_t t = e < 4 ? ta[e & 3] : tb[e & 3];
-        if (slot < TOPK) s_key[slot] = ((uint64_t)oct_half(wv, e) << 20) | (0xfffffu - t);
+        if (slot < TOPK) s_key[slot] = ((uint64_t)oct_half(wv, e) << 20) | (0xfffffu - tk.id(e));
         ++slot;
       }
       if (threadIdx.x == 0) s_cnt = nm;
       done = listed = true;
+    } else {
+      __syncthreads();  // the scratch is used again below
     }
   }
   const UnionScores src{sc, bmg, W};
@@ -1688,13 +1725,24 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
   const AttnLoads<TOP_KPW> L =
       attend_load<TOP_KPW>(kv_base<PAGED>(a, g), kv_lane_row<PAGED>(a, g, tk));
   SKV_TSB(9, 1);  // trace builds: the top-100 record gather is issued
-  // the output list, best first (member keys are distinct)
+  // the output list, best first (member keys are distinct): 8 threads per
+  // member count the keys above it (one thread per member took 1.8 us)
   int* out = a.top + j * TOPK;
-  if ((int)threadIdx.x < m) {
-    const uint64_t key = s_key[threadIdx.x];
-    out[count_above64(s_key, m, key)] = (int)(0xfffffu - (uint32_t)(key & 0xfffffu));
-  } else if ((int)threadIdx.x < TOPK) {
-    out[threadIdx.x] = -1;
+  static_assert(TOPK * 8 <= SEL_BLOCK, "8 threads per member");
+  {
+    const int i = threadIdx.x >> 3, part = threadIdx.x & 7;
+    const uint64_t key = s_key[min(i, TOPK - 1)];
+    int above = 0;
+#pragma unroll
+    for (int c = 0; c < (TOPK + 7) / 8; ++c) {
+      const int o = 8 * c + part;
+      above += o < m && s_key[min(o, TOPK - 1)] > key;
+    }
+    above += __builtin_amdgcn_update_dpp(0, above, 0xB1, 0xf, 0xf, false);   // quad_perm [1,0,3,2]
+    above += __builtin_amdgcn_update_dpp(0, above, 0x4E, 0xf, 0xf, false);   // quad_perm [2,3,0,1]
+    above += __builtin_amdgcn_update_dpp(0, above, 0x141, 0xf, 0xf, false);  // row_half_mirror
+    if (part == 0 && i < m) out[above] = (int)(0xfffffu - (uint32_t)(key & 0xfffffu));
+    if (part == 0 && i >= m && i < TOPK) out[i] = -1;
   }
   SKV_TS(13, 8);
   SKV_WAIT(L.kw[TOP_KPW - 1] ^ L.vw[TOP_KPW - 1]);  // trace builds: ... and has arrived

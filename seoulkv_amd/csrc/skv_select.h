@@ -34,7 +34,7 @@ struct SelectScratch {
   uint32_t hist4[16];
   int sel[2];
   int ntie;
-  int scan[SEL_WAVES + 1];
+  int scan[SEL_WAVES];
 };
 
 // Selection outcome: member(i) <=> ord > v || (ord == v && id <= idcut),

@@ -153,75 +153,160 @@ __device__ __forceinline__ void load_b(const QOperand* q, uint32_t b[4][4]) {
 
 // ============================================================ sparse SDPA
 // Attention of query head j = 4g + h over its KV group's FP8 [V || K] records
-// for the keys [sink | local | top-100] (softmax over all of them, scale 1/16).
-// The sink/local part depends only on Q: extra blocks of the k_select launch
-// compute it as 128-key slices (partial max, sum, unnormalised output), and
-// k_top100 attends the head's 100 selected keys and merges everything.
+// for the keys [sink | local | top-100] (softmax over all of them, scale 1/16;
+// logits and maxima in log2 units).  The sink/local part depends only on Q:
+// extra blocks of the k_select launch compute it as 256-key slices (partial
+// max, sum, unnormalised output), and k_top100 attends the head's 100
+// selected keys and merges everything.
+//
+// Bound by the vector instructions of one CU (16 waves, 4 per SIMD: each
+// instruction takes 16 cycles of the block), so a wave reads 4 keys per
+// 16-byte load, row r of 16 lanes holding key 4i + r, lane c its dims
+// 16c .. 16c + 15: a dot product is 16 FMAs and a 4-step row sum for 4 keys,
+// one exponential covers 4 keys, and the rows' outputs are summed by half-
+// and row-swaps that halve the values at each step.  (A key per wave
+// instruction, reduced over 64 lanes and its probability broadcast, took
+// about 35 instructions per key, here 16.  The select launch, which waited
+// for the sink/local slices: 6.5 -> 4.6 us at 512 centroids per head, 6.7 ->
+// 5.4 at 8192; k_top100 with the ranks of the output list below 9.2 -> 8.1.)
 constexpr int SDPA_WAVE_KEYS = 16;
 constexpr int DENSE_BLOCK_KEYS = (SEL_BLOCK / WAVE) * SDPA_WAVE_KEYS;
 static_assert(U2_MAX <= OCT_ITEMS && U1_MAX <= OCT_ITEMS, "unions fit the register selection");
 static_assert(DENSE_BLOCK_KEYS == DENSE_SLICE_KEYS && SEL_BLOCK / WAVE == ATTN_WAVES,
               "attention slices follow the selection block size");
+constexpr float ATTN_SCALE = 1.4426950408889634f / 16.f;  // log2(e) / sqrt(256)
 
-__device__ __forceinline__ void load_q4(const StepArgs& a, int j, float q[4]) {
-  const int lane = threadIdx.x & 63;
-  const uint2 qw = *reinterpret_cast<const uint2*>(a.q + j * D + 4 * lane);
-  q[0] = bf16_f32(qw.x & 0xffff); q[1] = bf16_f32(qw.x >> 16);
-  q[2] = bf16_f32(qw.y & 0xffff); q[3] = bf16_f32(qw.y >> 16);
+// This lane's 16 query dims (16 (lane % 16) ..) of head j.
+__device__ __forceinline__ void load_q16(const uint16_t* q, int j, float (&f)[16]) {
+  const uint4* row = reinterpret_cast<const uint4*>(q + j * D + 16 * (threadIdx.x & 15));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint4 w = row[i];
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[8 * i + 2 * e] = __uint_as_float(u[e] << 16);
+      f[8 * i + 2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
+    }
+  }
 }
 
-// One wave over up to KPW keys: lane b < KPW holds the token of key b in tk
-// (-1: none); lane l owns dims 4l..4l+3.  attend_load issues every record
-// load; attend_math (after any independent work) returns the wave's max
-// logit m, softmax sum l and unnormalised output o.
-template <int KPW>
+// Both halves (rows) of a pair of values exchanged: x + y, with a = sum over
+// the lane pairs 32 (16) apart of x in the lower half (even rows) and of y in
+// the upper half (odd rows).
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float half_sum(float x, float y) {
+  const u32x2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float row_pair_sum(float x, float y) {
+  const u32x2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float rows_max(float x) {  // over the 4 rows, every lane
+  u32x2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Sum or maximum over the 16 lanes of a row, in every lane of it: pairs,
+// quads, half rows, rows.
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov_f(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_sum_f(float v) {
+  v += dpp_mov_f<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_mov_f<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp_mov_f<0x141>(v);  // row_half_mirror
+  v += dpp_mov_f<0x140>(v);  // row_mirror
+  return v;
+}
+__device__ __forceinline__ float row_max_f(float v) {
+  v = fmaxf(v, dpp_mov_f<0xB1>(v));
+  v = fmaxf(v, dpp_mov_f<0x4E>(v));
+  v = fmaxf(v, dpp_mov_f<0x141>(v));
+  v = fmaxf(v, dpp_mov_f<0x140>(v));
+  return v;
+}
+
+// One wave over up to 4 I keys: rec[i] is the record index of key 4i + row of
+// this lane (-1: none).  attend_load issues every record load; attend_math
+// (after any independent work) returns the wave's max logit m, softmax sum l
+// and unnormalised output o of dims 16 (lane % 16) + 4 (lane / 16) + 0..3.
+template <int I>
 struct AttnLoads {
-  int t[KPW];
-  uint32_t kw[KPW], vw[KPW];
+  bool has[I];
+  uint4 k[I], v[I];
 };
 
-template <int KPW>
-__device__ __forceinline__ AttnLoads<KPW> attend_load(const uint8_t* __restrict__ kv, int tk) {
-  const int lane = threadIdx.x & 63;
-  AttnLoads<KPW> L;
+template <int I>
+__device__ __forceinline__ AttnLoads<I> attend_load(const uint8_t* __restrict__ kv,
+                                                    const int (&rec)[I]) {
+  const int c = threadIdx.x & 15;
+  AttnLoads<I> L;
 #pragma unroll
-  for (int b = 0; b < KPW; ++b) {
-    L.t[b] = __builtin_amdgcn_readlane(tk, b);
-    const uint8_t* rec = kv + (size_t)max(L.t[b], 0) * 512;
-    L.kw[b] = *reinterpret_cast<const uint32_t*>(rec + 256 + 4 * lane);
-    L.vw[b] = *reinterpret_cast<const uint32_t*>(rec + 4 * lane);
+  for (int i = 0; i < I; ++i) {
+    L.has[i] = rec[i] >= 0;
+    const uint8_t* p = kv + (size_t)max(rec[i], 0) * 512 + 16 * c;
+    L.k[i] = *reinterpret_cast<const uint4*>(p + 256);
+    L.v[i] = *reinterpret_cast<const uint4*>(p);
   }
   return L;
 }
 
-template <int KPW>
-__device__ __forceinline__ void attend_math(const AttnLoads<KPW>& L, const float q[4], float& m,
-                                            float& l, float o[4]) {
-  float logit[KPW];
+__device__ __forceinline__ void fp8x16_to_f32(uint4 w, float (&f)[16]) {
+  fp8x4_to_f32(w.x, f);
+  fp8x4_to_f32(w.y, f + 4);
+  fp8x4_to_f32(w.z, f + 8);
+  fp8x4_to_f32(w.w, f + 12);
+}
+
+template <int I>
+__device__ __forceinline__ void attend_math(const AttnLoads<I>& L, const float (&q)[16], float& m,
+                                            float& l, float (&o)[4]) {
+  float z[I];
+  float lm = -INFINITY;
 #pragma unroll
-  for (int b = 0; b < KPW; ++b) {
-    float kf[4];
-    fp8x4_to_f32(L.kw[b], kf);
-    logit[b] = q[0] * kf[0] + q[1] * kf[1] + q[2] * kf[2] + q[3] * kf[3];
+  for (int i = 0; i < I; ++i) {
+    float f[16];
+    fp8x16_to_f32(L.k[i], f);
+    float d0 = 0.f, d1 = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+      d0 = fmaf(q[e], f[e], d0);
+      d1 = fmaf(q[e + 1], f[e + 1], d1);
+    }
+    const float d = row_sum_f(d0 + d1) * ATTN_SCALE;
+    z[i] = L.has[i] ? d : -INFINITY;
+    lm = fmaxf(lm, z[i]);
   }
-#pragma unroll
-  for (int b = 0; b < KPW; ++b) logit[b] = wave_sum_f(logit[b]);
-  m = -INFINITY;
-#pragma unroll
-  for (int b = 0; b < KPW; ++b)
-    if (L.t[b] >= 0) m = fmaxf(m, logit[b] * 0.0625f);
+  m = rows_max(lm);
   l = 0.f;
-  o[0] = o[1] = o[2] = o[3] = 0.f;
+  float acc[16];
 #pragma unroll
-  for (int b = 0; b < KPW; ++b) {
-    if (L.t[b] < 0) continue;
-    const float p = __expf(logit[b] * 0.0625f - m);
-    float vf[4];
-    fp8x4_to_f32(L.vw[b], vf);
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int i = 0; i < I; ++i) {
+    const float x = __builtin_amdgcn_exp2f(z[i] - m);
+    const float p = L.has[i] ? x : 0.f;
     l += p;
+    // (an absent key read record 0, whose values may be NaN)
+    const uint32_t keep = L.has[i] ? ~0u : 0u;
+    float f[16];
+    fp8x16_to_f32(make_uint4(L.v[i].x & keep, L.v[i].y & keep, L.v[i].z & keep, L.v[i].w & keep), f);
 #pragma unroll
-    for (int d = 0; d < 4; ++d) o[d] += p * vf[d];
+    for (int e = 0; e < 16; ++e) acc[e] = fmaf(p, f[e], acc[e]);
   }
+  l = half_sum(l, l);
+  l = row_pair_sum(l, l);
+  // over the rows: lanes of the upper half keep dims 8 .. 15 of the 16, odd
+  // rows the upper 4 of those
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = half_sum(acc[e], acc[e + 8]);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = row_pair_sum(acc[e], acc[e + 4]);
 }
 
 struct AttnScratch {
@@ -232,40 +317,34 @@ static_assert(sizeof(AttnScratch) == ATTN_SCRATCH_BYTES, "attention scratch size
 
 // Publish a wave partial to LDS; after a barrier, merge_waves gives thread
 // d < 256 the block's (max, sum, output[d]).
-__device__ __forceinline__ void stash_wave(AttnScratch& s, float m, float l, const float o[4]) {
+__device__ __forceinline__ void stash_wave(AttnScratch& s, float m, float l, const float (&o)[4]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) {
     s.m[wave] = m;
     s.l[wave] = l;
   }
-#pragma unroll
-  for (int d = 0; d < 4; ++d) s.o[wave][4 * lane + d] = o[d];
+  *reinterpret_cast<float4*>(&s.o[wave][16 * (lane & 15) + 4 * (lane >> 4)]) =
+      make_float4(o[0], o[1], o[2], o[3]);
 }
 
+// Called by whole waves.  A wave without keys has m = -inf, l = o = 0 and
+// weight 0; lane w % 16 works out wave w's weight.
 __device__ __forceinline__ void merge_waves(const AttnScratch& s, int d, float& M, float& L,
                                             float& O) {
   constexpr int NW = SEL_BLOCK / WAVE;
-  // every LDS read issued before the first use (no per-wave branch); a wave
-  // without keys has m = -inf, l = o = 0 and weight exp(-inf) = 0
-  float mw[NW], lw[NW], ow[NW];
+  static_assert(NW == 16, "one row of lanes");
+  float ow[NW];  // every LDS read issued before the first use
 #pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    mw[w] = s.m[w];
-    lw[w] = s.l[w];
-    ow[w] = s.o[w][d];
-  }
-  M = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) M = fmaxf(M, mw[w]);
-  L = 0.f;
+  for (int w = 0; w < NW; ++w) ow[w] = s.o[w][d];
+  const float mw = s.m[threadIdx.x & 15], lw = s.l[threadIdx.x & 15];
+  M = row_max_f(mw);
+  const float x = __builtin_amdgcn_exp2f(mw - M);
+  const float sc = mw == -INFINITY ? 0.f : x;
+  L = row_sum_f(lw * sc);
   O = 0.f;
-  if (M == -INFINITY) return;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    const float sc = __expf(mw[w] - M);
-    L += lw[w] * sc;
-    O += ow[w] * sc;
-  }
+  for (int w = 0; w < NW; ++w)
+    O = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), w)), ow[w], O);
 }
 
 // Record base and per-lane record index of token tk (-1: none) of group g:
@@ -284,22 +363,26 @@ __device__ __forceinline__ int kv_lane_row(const StepArgs& a, int g, int tk) {
 // Dense slice r of query head j: keys r*256 .. r*256+255 of [sink | local].
 template <bool PAGED>
 __device__ __forceinline__ void dense_attend(const StepArgs& a, int blk, AttnScratch& s) {
+  constexpr int I = SDPA_WAVE_KEYS / 4;
   const int j = blk / a.dense_slices, r = blk % a.dense_slices, g = j / H;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ndense = a.sink + a.local;
-  float q[4];
-  load_q4(a, j, q);
-  int tk = -1;
-  const int i = r * DENSE_BLOCK_KEYS + wave * SDPA_WAVE_KEYS + lane;
-  if (lane < SDPA_WAVE_KEYS && i < ndense) tk = i < a.sink ? i : a.T - a.local + (i - a.sink);
-  float m, l, o[4];
+  int rec[I];
+#pragma unroll
+  for (int i = 0; i < I; ++i) {
+    const int n = r * DENSE_BLOCK_KEYS + wave * SDPA_WAVE_KEYS + 4 * i + (lane >> 4);
+    const int tk = n >= ndense ? -1 : n < a.sink ? n : a.T - a.local + (n - a.sink);
+    rec[i] = kv_lane_row<PAGED>(a, g, tk);
+  }
   // the slice's record gather (trace builds time it: issue, then arrival)
-  const AttnLoads<SDPA_WAVE_KEYS> L =
-      attend_load<SDPA_WAVE_KEYS>(kv_base<PAGED>(a, g), kv_lane_row<PAGED>(a, g, tk));
+  const AttnLoads<I> L = attend_load<I>(kv_base<PAGED>(a, g), rec);
+  float q[16];
+  load_q16(a.q, j, q);
   SKV_TSB(5, 1);
-  SKV_WAIT(L.kw[SDPA_WAVE_KEYS - 1] ^ L.vw[SDPA_WAVE_KEYS - 1]);
+  SKV_WAIT(L.k[I - 1].w ^ L.v[I - 1].w);
   SKV_TSW(5, 2);
-  attend_math<SDPA_WAVE_KEYS>(L, q, m, l, o);
+  float m, l, o[4];
+  attend_math<I>(L, q, m, l, o);
   stash_wave(s, m, l, o);
   __syncthreads();
   if (threadIdx.x < D) {
@@ -1546,6 +1629,7 @@ __global__ __launch_bounds__(US_BLOCK) void k_union_score(const int* count_word,
 // U1 position is set in any head's top-256 bitmap, so the members come out
 // in U1 order, which is U2's list order.
 constexpr int TOP_KPW = (TOPK + ATTN_WAVES - 1) / ATTN_WAVES;  // selected keys per wave
+constexpr int TOP_KEYS = (TOPK + 7) / 8 * 8;
 constexpr int DENSE_PREF = 2;  // sink/local partials prefetched per merge thread
 
 // Bits 8o .. 8o + 7 of the union of 4 bitmap rows of W words (octet o).
@@ -1593,7 +1677,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
   const int g = blockIdx.x / H, h = blockIdx.x % H, j = g * H + h;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __shared__ SelectScratch s;
-  __shared__ __align__(16) uint64_t s_key[TOPK];
+  __shared__ __align__(16) uint64_t s_key[TOP_KEYS];  // member keys; 0 past the members
   __shared__ __align__(16) uint32_t s_pos[TOPK];  // U1 positions (atomic-order paths)
   __shared__ int s_cnt;
   __shared__ int s_u2[SEL_WAVES];  // U2 members per wave's octets
@@ -1612,12 +1696,8 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
   }
   // loads independent of the selection, issued first: the query and the
   // sink/local partials (consumed only by the final merge)
-  float q[4];
-  {
-    const uint2 qw = *reinterpret_cast<const uint2*>(q_in + j * D + 4 * lane);
-    q[0] = bf16_f32(qw.x & 0xffff); q[1] = bf16_f32(qw.x >> 16);
-    q[2] = bf16_f32(qw.y & 0xffff); q[3] = bf16_f32(qw.y >> 16);
-  }
+  float q[16];
+  load_q16(q_in, j, q);
   const int d = threadIdx.x & (D - 1);
   const float* parts = dense_part + (size_t)j * dense_slices * (D + 2);
   float pm[DENSE_PREF], pl[DENSE_PREF], po[DENSE_PREF];
@@ -1629,6 +1709,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
     po[r] = has ? parts[r * (D + 2) + d] : 0.f;
   }
   if (threadIdx.x == 0) s_cnt = 0;
+  if (threadIdx.x < TOP_KEYS) s_key[threadIdx.x] = 0;  // (a barrier before any key is written)
   bool done = false, listed = false;  // listed: s_key is in U2 list order
   if (exact_select == 0) {  // n <= U1_MAX <= OCT_ITEMS: scores and IDs in registers
     const uint4 w[1] = {keep_octet(load_oct(sc, n), ubits)};
@@ -1715,40 +1796,42 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
     if ((int)threadIdx.x < m) s_key[rank] = key;
     __syncthreads();
   }
-  // attention over the members: wave w takes list entries w + 16 b; the
-  // record loads are issued before the output list is ranked
-  int tk = -1;
-  if (lane < TOP_KPW) {
-    const int i = wave + ATTN_WAVES * lane;
-    if (i < m) tk = (int)(0xfffffu - (uint32_t)(s_key[i] & 0xfffffu));
+  // attention over the members: wave w takes list entries w + 16 b
+  constexpr int I = (TOP_KPW + 3) / 4;
+  int rec[I];
+#pragma unroll
+  for (int i = 0; i < I; ++i) {
+    const int e = wave + ATTN_WAVES * (4 * i + (lane >> 4));
+    const int tk = (int)(0xfffffu - (uint32_t)(s_key[min(e, TOPK - 1)] & 0xfffffu));
+    rec[i] = kv_lane_row<PAGED>(a, g, e < m ? tk : -1);
   }
-  const AttnLoads<TOP_KPW> L =
-      attend_load<TOP_KPW>(kv_base<PAGED>(a, g), kv_lane_row<PAGED>(a, g, tk));
+  const AttnLoads<I> L = attend_load<I>(kv_base<PAGED>(a, g), rec);
   SKV_TSB(9, 1);  // trace builds: the top-100 record gather is issued
-  // the output list, best first (member keys are distinct): 8 threads per
-  // member count the keys above it (one thread per member took 1.8 us)
-  int* out = a.top + j * TOPK;
-  static_assert(TOPK * 8 <= SEL_BLOCK, "8 threads per member");
+  // the output list, best first (member keys are distinct), while the records
+  // arrive: 8 threads per member count the keys above it, every key read
+  // before the first is compared (one thread per member took 1.8 us; on the
+  // waves that the merge leaves idle, 4 threads per member, 2.0 us)
+  static_assert(TOPK * 8 <= SEL_BLOCK && TOP_KEYS % 8 == 0, "8 threads per member");
   {
     const int i = threadIdx.x >> 3, part = threadIdx.x & 7;
-    const uint64_t key = s_key[min(i, TOPK - 1)];
+    const uint64_t key = s_key[min(i, TOP_KEYS - 1)];
+    uint64_t other[TOP_KEYS / 8];
+#pragma unroll
+    for (int c = 0; c < TOP_KEYS / 8; ++c) other[c] = s_key[8 * c + part];
     int above = 0;
 #pragma unroll
-    for (int c = 0; c < (TOPK + 7) / 8; ++c) {
-      const int o = 8 * c + part;
-      above += o < m && s_key[min(o, TOPK - 1)] > key;
-    }
-    above += __builtin_amdgcn_update_dpp(0, above, 0xB1, 0xf, 0xf, false);   // quad_perm [1,0,3,2]
-    above += __builtin_amdgcn_update_dpp(0, above, 0x4E, 0xf, 0xf, false);   // quad_perm [2,3,0,1]
-    above += __builtin_amdgcn_update_dpp(0, above, 0x141, 0xf, 0xf, false);  // row_half_mirror
-    if (part == 0 && i < m) out[above] = (int)(0xfffffu - (uint32_t)(key & 0xfffffu));
-    if (part == 0 && i >= m && i < TOPK) out[i] = -1;
+    for (int c = 0; c < TOP_KEYS / 8; ++c) above += other[c] > key;  // (no member: 0)
+    above += __builtin_amdgcn_update_dpp(0, above, 0xB1, 0xf, 0xf, true);   // quad_perm [1,0,3,2]
+    above += __builtin_amdgcn_update_dpp(0, above, 0x4E, 0xf, 0xf, true);   // quad_perm [2,3,0,1]
+    above += __builtin_amdgcn_update_dpp(0, above, 0x141, 0xf, 0xf, true);  // row_half_mirror
+    if (part == 0 && i < TOPK)
+      a.top[j * TOPK + (i < m ? above : i)] = i < m ? (int)(0xfffffu - (uint32_t)(key & 0xfffffu)) : -1;
   }
   SKV_TS(13, 8);
-  SKV_WAIT(L.kw[TOP_KPW - 1] ^ L.vw[TOP_KPW - 1]);  // trace builds: ... and has arrived
+  SKV_WAIT(L.k[I - 1].w ^ L.v[I - 1].w);  // trace builds: ... and has arrived
   SKV_TSW(9, 2);
   float mw, lw, ow[4];
-  attend_math<TOP_KPW>(L, q, mw, lw, ow);
+  attend_math<I>(L, q, mw, lw, ow);
   stash_wave(att, mw, lw, ow);
   __syncthreads();
   SKV_TS(13, 9);
@@ -1766,25 +1849,24 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
 #pragma unroll
     for (int r = 0; r < DENSE_PREF; ++r) Mt = fmaxf(Mt, pm[r]);
     for (int r = DENSE_PREF; r < dense_slices; ++r) Mt = fmaxf(Mt, parts[r * (D + 2) + D]);
-    float Lt = 0.f, Ot = 0.f;
-    if (M != -INFINITY) {
-      const float sc0 = __expf(M - Mt);
-      Lt = Ls * sc0;
-      Ot = O * sc0;
-    }
+    // (a part without keys has max -inf and weight 0)
+    auto weight = [Mt](float x) {
+      const float f = __builtin_amdgcn_exp2f(x - Mt);
+      return x == -INFINITY ? 0.f : f;
+    };
+    const float sc0 = weight(M);
+    float Lt = Ls * sc0, Ot = O * sc0;
 #pragma unroll
     for (int r = 0; r < DENSE_PREF; ++r) {
-      if (pm[r] == -INFINITY) continue;
-      const float f = __expf(pm[r] - Mt);
-      Lt += pl[r] * f;
-      Ot += po[r] * f;
+      const float f = weight(pm[r]);
+      Lt = fmaf(pl[r], f, Lt);
+      Ot = fmaf(po[r], f, Ot);
     }
     for (int r = DENSE_PREF; r < dense_slices; ++r) {
-      const float mr = parts[r * (D + 2) + D];
-      if (mr == -INFINITY) continue;
-      const float f = __expf(mr - Mt);
-      Lt += parts[r * (D + 2) + D + 1] * f;
-      Ot += parts[r * (D + 2) + d] * f;
+      const float* pr = parts + r * (D + 2);
+      const float f = weight(pr[D]);
+      Lt = fmaf(pr[D + 1], f, Lt);
+      Ot = fmaf(pr[d], f, Ot);
     }
     const uint16_t ob = (uint16_t)bf16_rne(Ot / Lt);
     a.out[j * D + d] = ob;

@@ -130,6 +130,13 @@ int skv_bind_query_device(void *handle, const void *q_dev, void *producer_stream
  * step on the handle's stream.  No host synchronisation, no readback. */
 int skv_enqueue(void *handle);
 
+/* skv_bind_query and skv_enqueue in one call.  The query rides with the first
+ * kernel's arguments (no upload of its own) unless a staged append or a
+ * captured step needs one; it stays bound for later calls either way.  Under a
+ * caller's stream capture the captured step holds this query: capture
+ * skv_enqueue instead to replay with the query bound last. */
+int skv_run(void *handle, const uint16_t *q_bf16);
+
 /* Reference synchronize (api.py:104-107).  Waits for the stream and, if
  * status is non-NULL, stores the per-group device status words [4][8]:
  * 0 pool size, 1 error code (0, 4 pool above capacity, 5 pool below the

@@ -113,6 +113,7 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
         "skv_bind_query": (i32, [vp, vp]),
         "skv_bind_query_device": (i32, [vp, vp, vp]),
         "skv_enqueue": (i32, [vp]),
+        "skv_run": (i32, [vp, vp]),
         "skv_sync": (i32, [vp, vp]),
         "skv_output_device": (i32, [vp, ctypes.POINTER(vp)]),
         "skv_output_tiles_device": (i32, [vp, ctypes.POINTER(vp)]),
@@ -335,6 +336,14 @@ class Runtime:
 
     def enqueue(self) -> None:
         self._check(self.lib.skv_enqueue(self.handle), "enqueue")
+
+    def run(self, q: torch.Tensor) -> None:
+        """``bind_query(q)`` and ``enqueue()`` in one call; the query rides
+        with the step's first launch instead of an upload of its own."""
+        if q.device.type != "cpu" or q.dtype != torch.bfloat16 or q.numel() != 16 * D:
+            raise ValueError("expected a CPU BF16 Q with 16 x 256 elements")
+        q = q.contiguous()
+        self._check(self.lib.skv_run(self.handle, q.data_ptr()), "run")
 
     def synchronize(self) -> dict:
         st = np.zeros((G, 8), dtype=np.int32)

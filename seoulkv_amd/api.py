@@ -180,8 +180,9 @@ class SeoulKV4:
         if self._state is None:
             self._state = self._initialize(q)
             self._host_kv = None
-        self._bind_query(q)
-        return self._run_bound()
+        self._state.run(q)
+        self._generation += 1
+        return DecodeResult(self, self._generation)
 
     def append(self, k: torch.Tensor, v: torch.Tensor) -> None:
         """Append ``n`` decoded tokens to the cache: ``k``, ``v`` [4, n, 256]

@@ -507,9 +507,11 @@ __device__ __forceinline__ void fr_score(const StepArgs& a, int g, int tile, int
 // than one pass of the grid covers), every FR_WAVES * gridDim.x tiles after
 // it, with the next tile's loads in flight while one is scored.
 // APPEND (the step folds a host append, a.app_n > 0): block 0 of each group
-// also packs the appended tokens' FP8 records.
-template <bool LOOP, bool APPEND>
-__global__ __launch_bounds__(FR_BLOCK) void k_front(const uint16_t* __restrict__ q, StepArgs a) {
+// also packs the appended tokens' FP8 records.  BIND: q is the launch's own
+// copy of the query (front_query), which block 0 of each group writes to a.q
+// for the later kernels.
+template <bool LOOP, bool APPEND, bool BIND>
+__device__ __forceinline__ void front_body(const uint16_t* q, const StepArgs& a) {
   SKV_TSB(4, 0);
   SKV_TS(0, 0);
   const int g = blockIdx.y, nc = a.nc;
@@ -541,6 +543,8 @@ __global__ __launch_bounds__(FR_BLOCK) void k_front(const uint16_t* __restrict__
   }
   __shared__ __align__(16) QOperand sq;
   prep_operand(a, g, QV_RAW, &sq, qw);
+  if (BIND && blockIdx.x == 0 && threadIdx.x < H * WAVE)  // wave w holds head w
+    *reinterpret_cast<uint2*>(const_cast<uint16_t*>(a.q) + g * H * D + 4 * threadIdx.x) = qw;
   SKV_TS(0, 1);
   if (tile < ntiles) {
     uint32_t b[4][4];
@@ -588,6 +592,20 @@ __global__ __launch_bounds__(FR_BLOCK) void k_front(const uint16_t* __restrict__
                    bf16x4_to_fp8(make_uint2(w1.x, w1.y)), bf16x4_to_fp8(make_uint2(w1.z, w1.w)));
   }
   SKV_TSE(4);
+}
+
+template <bool LOOP, bool APPEND>
+__global__ __launch_bounds__(FR_BLOCK) void k_front(const uint16_t* __restrict__ q, StepArgs a) {
+  front_body<LOOP, APPEND, false>(q, a);
+}
+
+// The front of a step whose query was bound from host memory since the last
+// one: the 8 KiB query comes as a kernel argument, so the step needs no
+// upload of its own (an in-stream copy before the front kernel cost 3.6 us of
+// every step: 128K 55.5 -> 52.7 us, 8K 44 -> 41, a new query per step).
+template <bool LOOP>
+__global__ __launch_bounds__(FR_BLOCK) void k_front_bind(StepArgs a, QueryArg qa) {
+  front_body<LOOP, false, true>(qa.q, a);
 }
 
 __device__ __forceinline__ uint32_t same16(uint32_t o) { return o; }
@@ -1903,12 +1921,18 @@ static void launch_topk(const TopkArgs& t, size_t lds, hipStream_t st) {
 // Launch every kernel of one decode step on stream st.  If ev is non-NULL
 // (N_STEP_KERNELS + 1 events), ev[i] is recorded before kernel i and
 // ev[N_STEP_KERNELS] after the last one.
-void launch_kernel(const StepArgs& a, const StepWork& w, hipStream_t st, int k) {
+void launch_kernel(const StepArgs& a, const StepWork& w, hipStream_t st, int k,
+                   const QueryArg* query) {
   const int tiles_blocks = std::min((a.nc + FR_CENTROIDS - 1) / FR_CENTROIDS, FR_MAX_BLOCKS);
   const size_t bm_lds = (size_t)PL_BM_WORDS * 4;
   switch (k) {
     case 0: {
       const bool loop = tiles_blocks * FR_CENTROIDS < a.nc, app = a.app_n > 0;
+      if (query) {  // never with a folded append (its upload carries the query)
+        hipLaunchKernelGGL(loop ? k_front_bind<true> : k_front_bind<false>, dim3(tiles_blocks, G),
+                           dim3(FR_BLOCK), 0, st, a, *query);
+        break;
+      }
       const auto fn = loop ? (app ? k_front<true, true> : k_front<true, false>)
                            : (app ? k_front<false, true> : k_front<false, false>);
       hipLaunchKernelGGL(fn, dim3(tiles_blocks, G), dim3(FR_BLOCK), 0, st, a.q, a);
@@ -1991,7 +2015,9 @@ hipError_t step_kernel_lds(const StepArgs& a, const StepWork& w, int k, size_t* 
   if (k == 0) {  // every front variant
     for (const void* f : {reinterpret_cast<const void*>(&k_front<true, false>),
                           reinterpret_cast<const void*>(&k_front<false, true>),
-                          reinterpret_cast<const void*>(&k_front<false, false>)}) {
+                          reinterpret_cast<const void*>(&k_front<false, false>),
+                          reinterpret_cast<const void*>(&k_front_bind<true>),
+                          reinterpret_cast<const void*>(&k_front_bind<false>)}) {
       hipFuncAttributes attr2;
       const hipError_t e2 = hipFuncGetAttributes(&attr2, f);
       if (e2 != hipSuccess) return e2;
@@ -2003,10 +2029,11 @@ hipError_t step_kernel_lds(const StepArgs& a, const StepWork& w, int k, size_t* 
   return hipSuccess;
 }
 
-void launch_step(const StepArgs& a, const StepWork& w, hipStream_t st, hipEvent_t* ev) {
+void launch_step(const StepArgs& a, const StepWork& w, hipStream_t st, hipEvent_t* ev,
+                 const QueryArg* query) {
   for (int k = 0; k < N_STEP_KERNELS; ++k) {
     if (ev) (void)hipEventRecord(ev[k], st);
-    launch_kernel(a, w, st, k);
+    launch_kernel(a, w, st, k, k == 0 ? query : nullptr);
   }
   if (ev) (void)hipEventRecord(ev[N_STEP_KERNELS], st);
 }

@@ -863,9 +863,9 @@ int skv_bind_query_device(void* handle, const void* q_dev, void* producer_stream
   return SKV_OK;
 }
 
-int skv_enqueue(void* handle) {
-  Handle* h = static_cast<Handle*>(handle);
-  if (!h) return SKV_ESTATE;
+// One step; query (host memory, or NULL: the bound query in device memory)
+// travels with the front kernel's arguments.
+static int enqueue_step(Handle* h, const QueryArg* query) {
   if (!h->bound) return fail(h, SKV_ESTATE, "bind a query before enqueue");
   HIPCHK(h, hipSetDevice(h->device));
   // a pending host append: packed by this step's k_front (eager launches),
@@ -889,7 +889,7 @@ int skv_enqueue(void* handle) {
       }
       ++h->prof_steps;
     }
-    launch_step(h->a, h->w, h->stream, h->prof_ev);
+    launch_step(h->a, h->w, h->stream, h->prof_ev, query);
     h->prof_pending = true;
   } else if (h->use_graph) {
     if (!h->graph_exec) {  // capture the kernels once on a private stream
@@ -902,13 +902,34 @@ int skv_enqueue(void* handle) {
     }
     HIPCHK(h, hipGraphLaunch(h->graph_exec, h->stream));
   } else {
-    launch_step(h->a, h->w, h->stream, nullptr);
+    launch_step(h->a, h->w, h->stream, nullptr, query);
   }
   h->a.app_n = 0;  // later steps (and kernel timings) pack nothing
   h->a.app_src = nullptr;
   HIPCHK(h, hipGetLastError());
   h->ran = true;
   return SKV_OK;
+}
+
+int skv_enqueue(void* handle) {
+  Handle* h = static_cast<Handle*>(handle);
+  return h ? enqueue_step(h, nullptr) : SKV_ESTATE;
+}
+
+int skv_run(void* handle, const uint16_t* q) {
+  Handle* h = static_cast<Handle*>(handle);
+  if (!h) return SKV_ESTATE;
+  if (!q) return fail(h, SKV_EINVAL, "NULL query");
+  // a captured step takes no arguments, and a folded append travels with the
+  // query's own upload
+  if (h->use_graph || h->pend_n) {
+    if (const int rc = skv_bind_query(h, q)) return rc;
+    return enqueue_step(h, nullptr);
+  }
+  QueryArg arg;
+  memcpy(arg.q, q, sizeof arg.q);
+  h->bound = true;
+  return enqueue_step(h, &arg);
 }
 
 int skv_graph_mode(void* handle, int enable) {

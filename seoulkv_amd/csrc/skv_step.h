@@ -121,6 +121,11 @@ struct StepArgs {
                             // rows stay zero (cleared once with the workspace)
 };
 
+// A query passed by value to k_front_bind: [16][256] BF16.
+struct QueryArg {
+  alignas(16) uint16_t q[G * H * D];
+};
+
 struct TopkArgs {
   const uint16_t* scores;   // [G][H][stride] ordered
   const int* tokens;        // [G][stride]
@@ -168,10 +173,14 @@ extern const char* const kKernelNames[N_STEP_KERNELS];
 size_t topk_dynamic_lds(int lds_items);
 
 // Kernel k (0 .. N_STEP_KERNELS - 1, in step order) of one decode step.
-void launch_kernel(const StepArgs& a, const StepWork& w, hipStream_t st, int k);
+// query: the front kernel takes the query from here instead of a.q and stores
+// it there for the kernels after it.
+void launch_kernel(const StepArgs& a, const StepWork& w, hipStream_t st, int k,
+                   const QueryArg* query = nullptr);
 // Static and dynamic LDS bytes per block of step kernel k as launched.
 hipError_t step_kernel_lds(const StepArgs& a, const StepWork& w, int k, size_t* static_bytes,
                            size_t* dynamic_bytes);
-void launch_step(const StepArgs& a, const StepWork& w, hipStream_t st, hipEvent_t* ev);
+void launch_step(const StepArgs& a, const StepWork& w, hipStream_t st, hipEvent_t* ev,
+                 const QueryArg* query = nullptr);
 
 }  // namespace skv

@@ -60,7 +60,10 @@ struct FastScratch {
     alignas(16) uint64_t cand[CAND_CAP];  // ord << 40 | position
     struct {
       alignas(16) uint32_t hist_b[4096];
-      uint16_t tiles[4096];  // tiles listed by tiled_select
+      union {
+        uint16_t tiles[4096];  // tiles listed by tiled_select
+        alignas(16) uint32_t hist_c[4096];
+      };
     };
   };
   alignas(16) uint32_t tie[FS_TIE_RANK];  // read as uint4 by count_below

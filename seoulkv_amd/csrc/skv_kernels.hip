@@ -657,16 +657,17 @@ __device__ __forceinline__ void select_in_registers(const StepArgs& a, const uin
 // The same for nc <= NO x 8 x SEL_BLOCK centroids held as NO octets per
 // thread (octet o of thread t: centroids 8 (t + o SEL_BLOCK) ..): all three
 // rows are loaded at once, the threshold and the fine selection each run in
-// registers, so the longer lists need no tile maxima and no second load
-// round.  The fine selection ranks ties by centroid ID as IDs (octet order is
-// not position order); with more ties at its P-th score than that ranking
-// holds it returns false (the threshold is written) and the caller runs the
-// fine selection another way.
+// registers (octn_top), so the longer lists need no tile maxima and no second
+// load round.  Where a selection does not fit that path (block-uniform), it
+// runs over an LDS copy of its scores.
 template <int NO>
-__device__ __forceinline__ bool select_in_registers_n(const StepArgs& a, const uint16_t* lower,
+__device__ __forceinline__ void select_in_registers_n(const StepArgs& a, const uint16_t* lower,
                                                       const uint16_t* upper, const uint16_t* fine,
-                                                      int nc, int g, int h, FastScratch& fs,
-                                                      uint32_t* thr_out) {
+                                                      int nc, int g, int h, unsigned char* dyn,
+                                                      SelectScratch& s) {
+  FastScratch& fs = *reinterpret_cast<FastScratch*>(dyn);
+  uint16_t* so = reinterpret_cast<uint16_t*>(dyn);
+  uint32_t* selbm = a.selbm + (size_t)g * (nc / 32);
   const int t = threadIdx.x;
   const size_t row = ((size_t)g * H + h) * nc;
   // the lower bounds first: the threshold waits for them alone (the waits
@@ -680,29 +681,53 @@ __device__ __forceinline__ bool select_in_registers_n(const StepArgs& a, const u
     wf[o] = load_oct(fine + row + o * OCT_ITEMS, nc - o * OCT_ITEMS);
   }
   auto cid = [t](int b) { return (uint32_t)(8 * (t + (b >> 3) * SEL_BLOCK) + (b & 7)); };
+  auto pos = [](int i) { return (uint32_t)i; };
   fs_clear(fs.hist, fs.w[0]);
   fs_clear(fs.hist_b, fs.w[1]);
+  fs_clear(fs.hist_c, fs.w[1]);
   __syncthreads();
-  const OctResult r1 = octn_select<NO, TIE_VALUE>(wl, a.P[g], cid, fs.hist, fs.w[0], fs, 2);
-  const uint32_t thr = r1.sel.all ? 0u : r1.sel.v;
+  const OctResult r1 = octn_top<NO, TIE_VALUE>(wl, a.P[g], cid, fs.hist, fs.hist_b, fs, 2);
+  uint32_t thr = r1.sel.all ? 0u : r1.sel.v;
+  if (r1.ok) {
+    // the fine selection's item counts reuse the thread maxima's histogram
+    // (last read before the item counts' barriers; the maxima's barrier is next)
+    fs_clear(fs.hist, fs.w[0]);
+  } else {
+    __syncthreads();
+    load_lds_scores(so, lower + row, nc, same16);
+    __syncthreads();
+    const Selection sel = block_select(so, nc, a.P[g], pos, s);
+    thr = sel.all ? 0u : sel.v;
+    __syncthreads();
+    fs_clear(fs.hist, fs.w[0]);
+    fs_clear(fs.hist_c, fs.w[1]);
+    __syncthreads();
+  }
   if (t == 0) a.thr[g * H + h] = thr;
-  *thr_out = thr;
   SKV_TS(2, 6);
   uint4 wm[NO];
 #pragma unroll
   for (int o = 0; o < NO; ++o) wm[o] = MaskedScores::pick4(wf[o], wu[o], thr);
-  const OctResult r2 = octn_select<NO, TIE_ID>(wm, a.P[g], cid, fs.hist_b, fs.w[1], fs, 4);
-  if (!r2.ok) return false;  // block-uniform
-  // items 8u .. 8u+7 (u = t + o SEL_BLOCK) are byte u & 3 of bitmap word u >> 2
+  const OctResult r2 = octn_top<NO, TIE_ID>(wm, a.P[g], cid, fs.hist_c, fs.hist, fs, 4);
+  if (r2.ok) {
+    // items 8u .. 8u+7 (u = t + o SEL_BLOCK) are byte u & 3 of bitmap word u >> 2
 #pragma unroll
-  for (int o = 0; o < NO; ++o) {
-    uint32_t m = ((r2.mine >> (8 * o)) & 0xffu) << (8 * (t & 3));
-    m |= __shfl_xor(m, 1);
-    m |= __shfl_xor(m, 2);
-    if ((t & 3) == 0 && m) atomicOr(&a.selbm[(size_t)g * (nc / 32) + ((t + o * SEL_BLOCK) >> 2)], m);
+    for (int o = 0; o < NO; ++o) {
+      uint32_t m = ((r2.mine >> (8 * o)) & 0xffu) << (8 * (t & 3));
+      m |= __shfl_xor(m, 1);
+      m |= __shfl_xor(m, 2);
+      if ((t & 3) == 0 && m) atomicOr(&selbm[(t + o * SEL_BLOCK) >> 2], m);
+    }
+  } else {
+    __syncthreads();  // the register selection's scratch has been read
+    load_lds_masked(so, fine + row, upper + row, thr, nc);
+    __syncthreads();
+    const Selection sel = block_select(so, nc, a.P[g], pos, s);
+    for_scores(so, nc, [&](int c, uint32_t o) {
+      if (sel.member(o, (uint32_t)c)) atomicOr(&selbm[c >> 5], 1u << (c & 31));
+    });
   }
   SKV_TS(2, 15);
-  return true;
 }
 
 // The leading arguments repeat the fields of a that the selection blocks'
@@ -744,22 +769,7 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_select(const uint16_t* lower, con
   }
   __shared__ SelectScratch s;
   if constexpr (NO > 1) {  // launched for exact_select == 0 and nc <= NO x OCT_ITEMS only
-    uint32_t thr;
-    if (!select_in_registers_n<NO>(a, lower, upper, fine, nc, g, h,
-                                   *reinterpret_cast<FastScratch*>(dyn), &thr)) {
-      // more ties at the P-th fine score than the register ranking holds:
-      // the full selection over the LDS copy of the eligible fine scores
-      const size_t row = ((size_t)g * H + h) * nc;
-      uint16_t* so = reinterpret_cast<uint16_t*>(dyn);
-      __syncthreads();  // the register selection's scratch has been read
-      load_lds_masked(so, fine + row, upper + row, thr, nc);
-      __syncthreads();
-      const Selection sel = block_select(so, nc, a.P[g], [](int i) { return (uint32_t)i; }, s);
-      uint32_t* selbm = a.selbm + (size_t)g * (nc / 32);
-      for_scores(so, nc, [&](int c, uint32_t o) {
-        if (sel.member(o, (uint32_t)c)) atomicOr(&selbm[c >> 5], 1u << (c & 31));
-      });
-    }
+    select_in_registers_n<NO>(a, lower, upper, fine, nc, g, h, dyn, s);
     SKV_TSE(5);
     return;
   }

@@ -68,7 +68,7 @@ template <int NO, TieRule RULE, typename IdFn>
 __device__ __forceinline__ OctResult octn_select(const uint4 (&w)[NO], int k, IdFn id,
                                                  uint32_t* hist, SelWords& ws, FastScratch& s,
                                                  int ts = -1) {
-  static_assert(NO >= 1 && NO <= 4 && !(RULE == TIE_POS && NO > 1), "octets per thread");
+  static_assert(NO >= 1 && NO <= 2 && !(RULE == TIE_POS && NO > 1), "octets per thread");
   OctResult res;
   res.ok = true;
   res.mine = 0;
@@ -173,6 +173,103 @@ __device__ __forceinline__ OctResult octn_select(const uint4 (&w)[NO], int k, Id
   int slot = slot0;
   for (uint32_t rest = eq; rest; rest &= rest - 1)  // rank = number of smaller tied IDs
     if (count_below(s.tie, dr.ties, s.tie[slot++]) < need) gt |= rest & (0u - rest);
+  res.mine = gt;
+  return res;
+}
+
+// octn_select for k well below the 8 NO SEL_BLOCK items (NO = 2 or 4): the
+// k-th largest thread maximum is at most the k-th largest item (k threads hold
+// an item that reaches it), so only items from its bin's floor f up are
+// counted, by distance above f (4096 bins of one score step; a few hundred to
+// a few thousand LDS additions instead of one per item and a second pass for
+// the low digits, which were bound by the additions: threshold and fine
+// selection of 32672 centroids 14.9 -> REPL us).  hmax and hitem with their
+// words are cleared, as for octn_select.  ok = false, with nothing selected:
+// the k-th score lies 4095 or more steps above f, or too many ties: the
+// caller runs the full selection.
+template <int NO, TieRule RULE, typename IdFn>
+__device__ __forceinline__ OctResult octn_top(const uint4 (&w)[NO], int k, IdFn id, uint32_t* hmax,
+                                              uint32_t* hitem, FastScratch& s, int ts = -1) {
+  static_assert(RULE == TIE_VALUE || RULE == TIE_ID, "ties by ID");
+  OctResult res;
+  res.ok = true;
+  res.mine = 0;
+  res.sel.v = 0;
+  res.sel.idcut = 0xffffffffu;
+  res.sel.above = 0;
+  res.sel.all = false;
+  u32x4 wv[NO];
+  u16x2 mx = {0, 0};
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    wv[o] = u32x4{w[o].x, w[o].y, w[o].z, w[o].w};
+    const uint32_t u[4] = {w[o].x, w[o].y, w[o].z, w[o].w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) mx = __builtin_elementwise_max(mx, __builtin_bit_cast(u16x2, u[q]));
+  }
+  const uint32_t top = max((uint32_t)mx[0], (uint32_t)mx[1]);
+  if (top) atomicAdd(&hmax[top >> 4], 1u);
+  __syncthreads();
+  SKV_TS(ts, 1);
+  fs_rank_bin(hmax, s.w[0], k);
+  __syncthreads();
+  SKV_TS(ts, 2);
+  const int b1 = s.w[0].sel[0];
+  const uint32_t f = b1 > 0 ? (uint32_t)b1 << 4 : 1u;  // 1: every valid item
+#pragma unroll
+  for (int o = 0; o < NO; ++o)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t x = oct_half(wv[o], e);
+      if (x >= f) atomicAdd(&hitem[min(x - f, 4095u)], 1u);
+    }
+  __syncthreads();
+  SKV_TS(ts, 3);
+  fs_rank_bin(hitem, s.w[1], k);
+  __syncthreads();
+  const int bin = s.w[1].sel[0];
+  uint32_t v = 1;
+  int need = 0, ties = 0;
+  if (bin < 0) {  // fewer than k valid items (f = 1): all of them are members
+    res.sel.all = true;
+    res.sel.above = s.w[1].sel[2];
+  } else {
+    if (bin == 4095) {
+      res.ok = false;
+      return res;
+    }
+    v = f + (uint32_t)bin;
+    res.sel.v = v;
+    res.sel.above = s.w[1].sel[1];
+    need = k - res.sel.above;
+    ties = (int)hitem[bin];
+  }
+  if (RULE == TIE_VALUE) return res;
+  uint32_t gt = 0, eq = 0;
+#pragma unroll
+  for (int o = 0; o < NO; ++o)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t x = oct_half(wv[o], e);
+      gt |= (uint32_t)(x > v) << (8 * o + e);
+      eq |= (uint32_t)(x == v) << (8 * o + e);
+    }
+  if (need >= ties) {  // (also when all are members)
+    res.mine = gt | eq;
+    return res;
+  }
+  if (ties > FS_TIE_RANK) {
+    res.ok = false;
+    return res;
+  }
+  const int c = __popc(eq);
+  const int slot0 = c ? atomicAdd(&s.w[1].ntie, c) : 0;
+  int slot = slot0;
+  for (uint32_t rest = eq; rest; rest &= rest - 1) s.tie[slot++] = id(__ffs(rest) - 1);
+  __syncthreads();
+  slot = slot0;
+  for (uint32_t rest = eq; rest; rest &= rest - 1)  // rank = number of smaller tied IDs
+    if (count_below(s.tie, ties, s.tie[slot++]) < need) gt |= rest & (0u - rest);
   res.mine = gt;
   return res;
 }

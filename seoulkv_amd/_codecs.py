@@ -36,7 +36,7 @@ QUERY_FIELDS = frozenset({"q", "query_hash", "coarse_ids", "head_mask"})
 def fingerprint(t: torch.Tensor) -> str:
     """SHA-256 of the tensor's raw bytes (reference ``_codecs/index.py:19-22``)."""
     raw = t.contiguous().view(torch.uint8).cpu().numpy()
-    return hashlib.sha256(raw.tobytes()).hexdigest()
+    return hashlib.sha256(raw).hexdigest()  # read in place: no copy of the keys
 
 
 def pack2(codes: torch.Tensor) -> torch.Tensor:

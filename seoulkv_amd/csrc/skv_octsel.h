@@ -183,7 +183,7 @@ __device__ __forceinline__ OctResult octn_select(const uint4 (&w)[NO], int k, Id
 // counted, by distance above f (4096 bins of one score step; a few hundred to
 // a few thousand LDS additions instead of one per item and a second pass for
 // the low digits, which were bound by the additions: threshold and fine
-// selection of 32672 centroids 14.9 -> REPL us).  hmax and hitem with their
+// selection of 32672 centroids 15.4 -> 11.5 us).  hmax and hitem with their
 // words are cleared, as for octn_select.  ok = false, with nothing selected:
 // the k-th score lies 4095 or more steps above f, or too many ties: the
 // caller runs the full selection.

@@ -314,7 +314,8 @@ __device__ __forceinline__ float2* dense_stats(float* part, int nb) {
 // three pairs in 4 waves of 512, spilled.)  Whole call with the merge, back
 // to back, against V sums on the vector ALUs (half of every SIMD's cycles)
 // with the query formed by every wave: T = 1000 16.6 -> 8.5 us, 40009 27 ->
-// 21, 131072 54.8 -> 47.1, 2^20 374 -> 310 (6.9 TB/s).
+// 21, 131072 54.8 -> 47.1, 2^20 374 -> 310 (6.9 TB/s); the reload below took
+// the middle two to 18 and 43-45 later.
 // The arguments are DenseArgs' fields as scalars, preloaded at dispatch: the
 // first loads need not wait for an argument block.
 template <bool PAGED>
@@ -366,11 +367,9 @@ __global__ __launch_bounds__(DN_BLOCK) void k_dense(const uint16_t* q, const uin
   const bool ragged = n > 0 && key0(n - 1) + 2 * DN_TILE > T;
   const int whole = n - (ragged ? 1 : 0);
   auto load_k = [&](DnPair& x, int i) {
-    i = min(i, whole - 1);  // (branch-free: past the end the last pair again, unused)
     dn_load_k<false>(x, tile0(i), tile1(i), 0, 0, lane);
   };
   auto load_v = [&](DnPair& x, int i) {
-    i = min(i, whole - 1);
     dn_load_v<false>(x, tile0(i), tile1(i), 0, 0, lane);
   };
   DnPair x;
@@ -388,11 +387,17 @@ __global__ __launch_bounds__(DN_BLOCK) void k_dense(const uint16_t* q, const uin
   float m = -INFINITY, l = 0.f;  // running max / this lane's sum of head col / 4
 
   // each half of the pair's registers is reloaded once it is used; the other
-  // waves of the CU cover the rest of the latency
+  // waves of the CU cover the rest of the latency.  No reload after the last
+  // pair: reading it again instead of branching fetched its streamed V half
+  // from memory once more, 290 MB for 268 MB at T = 131072, where a wave has
+  // 5.3 pairs (24577 keys 17.0 -> 14.6 us, 40009 20.3 -> 18.2, 131072 44.4 ->
+  // 43.3, 2^20 the same; with the branch on V alone 15.2, 19.5, 43.1).
 #pragma nounroll
   for (int i = 0; i < whole; ++i) {
-    dn_pair<false>(x, key0(i), T, lane, s_q, zc, o, m, l, [&] { load_k(x, i + 1); });
-    load_v(x, i + 1);
+    dn_pair<false>(x, key0(i), T, lane, s_q, zc, o, m, l, [&] {
+      if (i + 1 < whole) load_k(x, i + 1);
+    });
+    if (i + 1 < whole) load_v(x, i + 1);
   }
   if (ragged) {
     const int i = n - 1;

@@ -144,15 +144,24 @@ int skv_run(void *handle, const uint16_t *q_bf16);
  * 6 postings scanned, 7 full-selection bits (see skv_select_mode). */
 int skv_sync(void *handle, int32_t *status);
 
-/* Device pointer of the output [16][256] BF16 (valid until skv_destroy;
- * overwritten by the next skv_enqueue). */
+/* Device pointer of the output [16][256] BF16 (valid until skv_destroy, or
+ * while a hold lasts: skv_output_hold; overwritten by the next skv_enqueue). */
 int skv_output_device(void *handle, void **dev_ptr);
 
 /* Device pointer of the same output in the reference's per-KV-head layout
  * (DecodeResult.device_tensors, result.py:25-28): [4][1][32][4][256] BF16,
  * query head 4g + h at [g][0][h][h], every other row zero.  Written by each
- * skv_enqueue with the compact output; valid until skv_destroy. */
+ * skv_enqueue with the compact output; valid as skv_output_device's. */
 int skv_output_tiles_device(void *handle, void **dev_ptr);
+
+/* A hold on the memory behind skv_output_device, skv_output_tiles_device and
+ * skv_dense_output_device: it stays allocated (about 0.3 MiB, with the last
+ * values written) until the hold is released, also past skv_destroy, which
+ * frees everything else.  Each hold is released once, from any thread, after
+ * the work that reads the outputs has been enqueued.  The reference leaves
+ * views of a closed instance to TT-NN's own reference counts. */
+int skv_output_hold(void *handle, void **hold);
+void skv_output_release(void *hold);
 
 /* Reference DecodeResult.to_torch (result.py:30-38): sync + copy [16][256]. */
 int skv_read_output(void *handle, uint16_t *host_out);
@@ -288,7 +297,8 @@ const char *skv_kernel_name(int i);
 /* Reference metadata (_runtime.py:197-454), as a JSON text. */
 const char *skv_metadata(void *handle);
 
-/* Releases every device buffer of the handle (reference close, api.py:128-137). */
+/* Releases every device buffer of the handle (reference close, api.py:128-137);
+ * its outputs when no hold on them is left. */
 void skv_destroy(void *handle);
 
 /* Text of the last error of this handle (or of the last failed create when

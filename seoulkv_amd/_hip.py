@@ -117,6 +117,8 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
         "skv_sync": (i32, [vp, vp]),
         "skv_output_device": (i32, [vp, ctypes.POINTER(vp)]),
         "skv_output_tiles_device": (i32, [vp, ctypes.POINTER(vp)]),
+        "skv_output_hold": (i32, [vp, ctypes.POINTER(vp)]),
+        "skv_output_release": (None, [vp]),
         "skv_read_output": (i32, [vp, vp]),
         "skv_debug_ids": (i32, [vp, vp]),
         "skv_read_stage": (i32, [vp, i32, i32, vp, i64, ctypes.POINTER(i64)]),
@@ -228,6 +230,24 @@ def index_desc(index, *, pool_min: int, pool_capacity: int | None, debug: bool,
     return desc, keep
 
 
+class OutputMemory:
+    """A hold on a runtime's output buffers (``skv_output_hold``): they stay
+    allocated while this object lives, also past the runtime's ``close``."""
+
+    def __init__(self, lib, handle):
+        self._lib, self._hold = lib, None
+        hold = ctypes.c_void_p()
+        code = lib.skv_output_hold(handle, ctypes.byref(hold))
+        if code != 0:
+            raise RuntimeError(f"output hold failed ({ERRORS.get(code, code)})")
+        self._hold = hold
+
+    def __del__(self):
+        hold, self._hold = self._hold, None
+        if hold is not None:
+            self._lib.skv_output_release(hold)
+
+
 class Runtime:
     """One device instance of the decode path (the reference's ``state``)."""
 
@@ -271,6 +291,7 @@ class Runtime:
             msg = self.lib.skv_last_error(None).decode()
             raise RuntimeError(f"skv_create failed ({ERRORS.get(code, code)}): {msg}")
         self.handle = handle
+        self.output = OutputMemory(self.lib, handle)  # outlives close()
         self.stream = int(stream) if stream else None  # the caller's stream (else the library's)
         self.device = int(device)
         self.nc = desc.n_centroids
@@ -356,12 +377,14 @@ class Runtime:
         return torch.from_numpy(out.view(np.int16)).view(torch.bfloat16).reshape(1, 1, 16, D)
 
     def output_device_ptr(self) -> int:
+        """Device [16][256] BF16 output; a view of it keeps ``self.output``."""
         p = ctypes.c_void_p()
         self._check(self.lib.skv_output_device(self.handle, ctypes.byref(p)), "output")
         return int(p.value)
 
     def output_tiles_device_ptr(self) -> int:
-        """Device [4][1][32][4][256] BF16 output in the reference's layout."""
+        """Device [4][1][32][4][256] BF16 output in the reference's layout; a
+        view of it keeps ``self.output``."""
         p = ctypes.c_void_p()
         self._check(self.lib.skv_output_tiles_device(self.handle, ctypes.byref(p)), "output")
         return int(p.value)
@@ -471,6 +494,8 @@ class Runtime:
         return dict(zip(names, ms.tolist())), steps.value
 
     def close(self) -> None:
+        """Release every device buffer but the outputs, which go with this
+        object and the views that hold ``output``."""
         if getattr(self, "handle", None):
             self.lib.skv_destroy(self.handle)
             self.handle = None

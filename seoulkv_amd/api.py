@@ -259,6 +259,16 @@ class SeoulKV4:
             self._release_pages()
             self._state = self._host_kv = self._index = None
 
+    def __del__(self):
+        # A dropped instance gives its device buffers back at once, also while
+        # a view of its output keeps the runtime object (and the outputs).
+        state = getattr(self, "_state", None)
+        if state is not None:
+            try:
+                state.close()
+            except Exception:
+                pass
+
     def __enter__(self):
         self._require_open()
         return self

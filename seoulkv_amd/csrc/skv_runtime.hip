@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -54,6 +55,20 @@ constexpr int APPEND_CHUNK = 256;   // tokens per host-append staging round
 constexpr int Q_RING = 16;          // query staging slots (host run-ahead, in steps)
 constexpr int Q_MARK = 8;           // uploads per completion event of the staging ring
 
+// A handle's output buffers, in a device allocation of their own: shared by
+// the handle and the callers of skv_output_hold, freed with the last of them,
+// so a view of an output never outlives its memory and never keeps the
+// handle's caches allocated.
+struct OutputMem {
+  std::atomic<int> refs{1};
+  void* mem = nullptr;
+};
+void release_output(OutputMem* o) {
+  if (!o || o->refs.fetch_sub(1) != 1) return;
+  if (o->mem) (void)hipFree(o->mem);
+  delete o;
+}
+
 constexpr int DEV_OK_SLOTS = 8;
 struct DevRange {
   uintptr_t lo, hi;
@@ -89,6 +104,7 @@ struct Handle {
   hipEvent_t steps_done = nullptr, q_ready = nullptr;
   void* static_mem = nullptr;
   void* work_mem = nullptr;
+  OutputMem* out_mem = nullptr;
   size_t static_bytes = 0, work_bytes = 0;
   StepArgs a{};
   StepWork w{};
@@ -355,6 +371,7 @@ void skv_destroy(void* handle) {
     if (e) (void)hipEventDestroy(e);
   if (h->static_mem) (void)hipFree(h->static_mem);
   if (h->work_mem) (void)hipFree(h->work_mem);
+  release_output(h->out_mem);
   if (h->own_stream && h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }
@@ -596,15 +613,11 @@ static int create_impl(const skv_index_desc* ix, const uint16_t* k_bf16, const u
     a.s8 = (uint16_t*)ar.take((size_t)G * H * U1_MAX * 2);
     a.top = (int*)ar.take(G * H * TOPK * 4);
     a.status = (int*)ar.take(G * ST_WORDS * 4);
-    a.out = (uint16_t*)ar.take(16 * D * 2);
-    a.out_tiles = (uint16_t*)ar.take((size_t)G * 32 * H * D * 2);
     a.bm_u1 = (uint64_t*)ar.take((size_t)G * H * words1 * 8);
     a.bm_u2 = (uint64_t*)ar.take((size_t)G * H * words2 * 8);
     h->dn.part = (float*)ar.take((size_t)G * DN_TARGET_BLOCKS * H * (D + 2) * 4);  // any T
-    h->dn.out = (uint16_t*)ar.take(16 * D * 2);
   };
   plan_work(wk);
-  h->work_bytes = wk.used;
   if (hipMalloc(&h->work_mem, wk.used) != hipSuccess) {
     fail(h, SKV_ENOMEM, "cannot allocate %zu bytes of device workspace", wk.used);
     return bail(SKV_ENOMEM);
@@ -612,11 +625,30 @@ static int create_impl(const skv_index_desc* ix, const uint16_t* k_bf16, const u
   wk.base = (char*)h->work_mem;
   wk.used = 0;
   plan_work(wk);
+  // ---- outputs (OutputMem)
+  Arena om;
+  auto plan_out = [&](Arena& ar) {
+    a.out = (uint16_t*)ar.take(16 * D * 2);
+    a.out_tiles = (uint16_t*)ar.take((size_t)G * 32 * H * D * 2);
+    h->dn.out = (uint16_t*)ar.take(16 * D * 2);
+  };
+  plan_out(om);
+  const size_t out_bytes = om.used;
+  h->out_mem = new OutputMem();
+  if (hipMalloc(&h->out_mem->mem, out_bytes) != hipSuccess) {
+    fail(h, SKV_ENOMEM, "cannot allocate %zu bytes of device output", out_bytes);
+    return bail(SKV_ENOMEM);
+  }
+  om.base = (char*)h->out_mem->mem;
+  om.used = 0;
+  plan_out(om);
+  h->work_bytes = wk.used + out_bytes;
   h->dn.kv8 = a.kv8;
   h->dn.table = a.kv_table;
   h->dn.shift = a.kv_shift;
   h->dn.q = a.q;
-  if (hipMemsetAsync(h->work_mem, 0, h->work_bytes, h->stream) != hipSuccess) {
+  if (hipMemsetAsync(h->work_mem, 0, wk.used, h->stream) != hipSuccess ||
+      hipMemsetAsync(h->out_mem->mem, 0, out_bytes, h->stream) != hipSuccess) {
     fail(h, SKV_EHIP, "workspace clear failed");
     return bail(SKV_EHIP);
   }
@@ -1222,6 +1254,16 @@ int skv_output_tiles_device(void* handle, void** dev_ptr) {
   *dev_ptr = h->a.out_tiles;
   return SKV_OK;
 }
+
+int skv_output_hold(void* handle, void** hold) {
+  Handle* h = static_cast<Handle*>(handle);
+  if (!h || !hold) return SKV_EINVAL;
+  h->out_mem->refs.fetch_add(1);
+  *hold = h->out_mem;
+  return SKV_OK;
+}
+
+void skv_output_release(void* hold) { release_output(static_cast<OutputMem*>(hold)); }
 
 int skv_read_output(void* handle, uint16_t* host_out) {
   Handle* h = static_cast<Handle*>(handle);

@@ -56,12 +56,13 @@ class GroupOutput:
 
     def device_view(self) -> torch.Tensor:
         """Device BF16 [1, 32, 4, 256] view of this KV head's tile of the
-        library's padded output buffer (valid until the next enqueue)."""
+        library's padded output buffer (until the next enqueue; past the
+        runtime's close, its last output)."""
         from seoulkv_amd.result import _DeviceArray
 
         raw = torch.as_tensor(
             _DeviceArray(self._runtime.output_tiles_device_ptr(), (4,) + self.shape, "<i2",
-                         self._runtime),
+                         self._runtime.output),
             device=f"cuda:{self._runtime.device}",
         ).view(torch.bfloat16)
         return raw[self.slot]

@@ -20,8 +20,9 @@ import torch
 class _DeviceArray:
     """__cuda_array_interface__ wrapper of a raw device pointer.  ``owner``
     (whose memory it is) lives as long as the wrapper, which PyTorch keeps for
-    as long as a tensor over it: a view outlives the instance it was taken
-    from being dropped (not its ``close()``)."""
+    as long as a tensor over it.  For a view of an output that is the runtime
+    or its ``output``: the 0.3 MiB of outputs outlive the instance being
+    dropped or closed, and nothing else of it does."""
 
     def __init__(self, ptr: int, shape, typestr: str, owner=None):
         self.owner = owner
@@ -53,7 +54,8 @@ class DecodeResult:
     def device_tensors(self) -> tuple:
         """Per KV group BF16 [1, 32, 4, 256] device views (query head 4g + h
         at [0, h, h]).  Call ``synchronize`` on the owner before reading
-        them; do not retain across close."""
+        them.  Every step overwrites them; past the owner's close they hold
+        its last output."""
         owner = self._owner()
         state = owner._require_initialized()
         ptr = state.output_tiles_device_ptr()

@@ -271,7 +271,8 @@ int skv_profile(void *handle, int enable);
  * the token top-k scores never held in LDS, so their in-memory radix passes
  * run at every pool size; 0 restores the default.  Status word 7 of each group (see skv_sync)
  * records, one bit per stage (1 thresh, 2 fine select, 4 top-1600, 8 top-256,
- * 16 top-100), which selections of the last step took the full path. */
+ * 16 top-100), which selections of the last step missed their sampled cut (or, at 8K-32K
+ * centroids, the bound from their thread maxima) and ran over every item. */
 int skv_select_mode(void *handle, int exact);
 
 /* Launch mode (no counterpart in the reference, whose programs are enqueued

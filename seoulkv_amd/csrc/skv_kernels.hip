@@ -658,8 +658,11 @@ __device__ __forceinline__ void select_in_registers(const StepArgs& a, const uin
 // thread (octet o of thread t: centroids 8 (t + o SEL_BLOCK) ..): all three
 // rows are loaded at once, the threshold and the fine selection each run in
 // registers (octn_top), so the longer lists need no tile maxima and no second
-// load round.  Where a selection does not fit that path (block-uniform), it
-// runs over an LDS copy of its scores.
+// load round.  Where octn_top's bound says too little (block-uniform: probe
+// budgets past 1024, few eligible centroids, a wide gap in the scores) the
+// two-pass octn_select takes the same registers; only a fine selection with
+// more than FS_TIE_RANK ties runs over an LDS copy of its scores.  Both are
+// recorded in ST_FULLSEL.
 template <int NO>
 __device__ __forceinline__ void select_in_registers_n(const StepArgs& a, const uint16_t* lower,
                                                       const uint16_t* upper, const uint16_t* fine,
@@ -686,29 +689,40 @@ __device__ __forceinline__ void select_in_registers_n(const StepArgs& a, const u
   fs_clear(fs.hist_b, fs.w[1]);
   fs_clear(fs.hist_c, fs.w[1]);
   __syncthreads();
-  const OctResult r1 = octn_top<NO, TIE_VALUE>(wl, a.P[g], cid, fs.hist, fs.hist_b, fs, 2);
-  uint32_t thr = r1.sel.all ? 0u : r1.sel.v;
-  if (r1.ok) {
-    // the fine selection's item counts reuse the thread maxima's histogram
-    // (last read before the item counts' barriers; the maxima's barrier is next)
-    fs_clear(fs.hist, fs.w[0]);
-  } else {
-    __syncthreads();
-    load_lds_scores(so, lower + row, nc, same16);
-    __syncthreads();
-    const Selection sel = block_select(so, nc, a.P[g], pos, s);
-    thr = sel.all ? 0u : sel.v;
+  const int P = a.P[g];
+  uint32_t missed = 0;  // ST_FULLSEL bits
+  OctResult r1;
+  r1.ok = false;
+  if (P <= SEL_BLOCK) r1 = octn_top<NO, TIE_VALUE>(wl, P, cid, fs.hist, fs.hist_b, fs, 2);
+  if (!r1.ok) {
+    missed |= FS_THRESH;
     __syncthreads();
     fs_clear(fs.hist, fs.w[0]);
-    fs_clear(fs.hist_c, fs.w[1]);
     __syncthreads();
+    r1 = octn_select<NO, TIE_VALUE>(wl, P, cid, fs.hist, fs.w[0], fs, 2);
+    __syncthreads();  // every wave has read its counts
   }
+  const uint32_t thr = r1.sel.all ? 0u : r1.sel.v;
+  // the fine selection's item counts reuse the thread maxima's histogram
+  // (last read before the item counts' barriers; the maxima's barrier is next)
+  fs_clear(fs.hist, fs.w[0]);
   if (t == 0) a.thr[g * H + h] = thr;
   SKV_TS(2, 6);
   uint4 wm[NO];
 #pragma unroll
   for (int o = 0; o < NO; ++o) wm[o] = MaskedScores::pick4(wf[o], wu[o], thr);
-  const OctResult r2 = octn_top<NO, TIE_ID>(wm, a.P[g], cid, fs.hist_c, fs.hist, fs, 4);
+  OctResult r2;
+  r2.ok = false;
+  r2.sel.v = 0;
+  if (P <= SEL_BLOCK) r2 = octn_top<NO, TIE_ID>(wm, P, cid, fs.hist_c, fs.hist, fs, 4);
+  if (!r2.ok) missed |= FS_FINE;
+  if (!r2.ok && r2.sel.v == 0) {
+    __syncthreads();
+    fs_clear(fs.hist, fs.w[0]);
+    __syncthreads();
+    r2 = octn_select<NO, TIE_ID>(wm, P, cid, fs.hist, fs.w[0], fs, 4);
+  }
+  if (missed && t == 0) atomicOr(&a.status[g * ST_WORDS + ST_FULLSEL], missed);
   if (r2.ok) {
     // items 8u .. 8u+7 (u = t + o SEL_BLOCK) are byte u & 3 of bitmap word u >> 2
 #pragma unroll
@@ -722,7 +736,7 @@ __device__ __forceinline__ void select_in_registers_n(const StepArgs& a, const u
     __syncthreads();  // the register selection's scratch has been read
     load_lds_masked(so, fine + row, upper + row, thr, nc);
     __syncthreads();
-    const Selection sel = block_select(so, nc, a.P[g], pos, s);
+    const Selection sel = block_select(so, nc, P, pos, s);
     for_scores(so, nc, [&](int c, uint32_t o) {
       if (sel.member(o, (uint32_t)c)) atomicOr(&selbm[c >> 5], 1u << (c & 31));
     });

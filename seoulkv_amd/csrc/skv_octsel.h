@@ -38,7 +38,8 @@ __device__ __forceinline__ uint4 load_oct(const uint16_t* __restrict__ row, int 
 struct OctResult {
   Selection sel;  // v (k-th best score), above (count scoring > v), all
   uint32_t mine;  // member bits of this thread's items (bit 8o + e = item e of octet o)
-  bool ok;        // false: too many ties at v to rank here (use the full path)
+  bool ok;        // false: too many ties at v to rank here (use the full path), or,
+                  // octn_top only, no v found (sel.v = 0: use octn_select)
 };
 
 // How items tied at the k-th score are ranked.
@@ -68,7 +69,7 @@ template <int NO, TieRule RULE, typename IdFn>
 __device__ __forceinline__ OctResult octn_select(const uint4 (&w)[NO], int k, IdFn id,
                                                  uint32_t* hist, SelWords& ws, FastScratch& s,
                                                  int ts = -1) {
-  static_assert(NO >= 1 && NO <= 2 && !(RULE == TIE_POS && NO > 1), "octets per thread");
+  static_assert(NO >= 1 && NO <= 4 && !(RULE == TIE_POS && NO > 1), "octets per thread");
   OctResult res;
   res.ok = true;
   res.mine = 0;
@@ -184,9 +185,14 @@ __device__ __forceinline__ OctResult octn_select(const uint4 (&w)[NO], int k, Id
 // a few thousand LDS additions instead of one per item and a second pass for
 // the low digits, which were bound by the additions: threshold and fine
 // selection of 32672 centroids 15.4 -> 11.5 us).  hmax and hitem with their
-// words are cleared, as for octn_select.  ok = false, with nothing selected:
-// the k-th score lies 4095 or more steps above f, or too many ties: the
-// caller runs the full selection.
+// words are cleared, as for octn_select.  ok = false, with nothing selected
+// and sel.v = 0, where the bound says too little and octn_select has to run:
+// fewer than k threads hold an item (always for k > SEL_BLOCK; items are then
+// not counted, all would land above the last step), or the k-th score lies
+// 4095 or more steps above f.  (Select launch with a budget of 2048 out of
+// 10240 / 24576 centroids 10.5 / 16.5 us; counting the items all the same, on
+// one bin, and selecting over LDS afterwards 36.4 / 54.8.)  ok = false with
+// sel.v: too many ties.
 template <int NO, TieRule RULE, typename IdFn>
 __device__ __forceinline__ OctResult octn_top(const uint4 (&w)[NO], int k, IdFn id, uint32_t* hmax,
                                               uint32_t* hitem, FastScratch& s, int ts = -1) {
@@ -215,7 +221,11 @@ __device__ __forceinline__ OctResult octn_top(const uint4 (&w)[NO], int k, IdFn 
   __syncthreads();
   SKV_TS(ts, 2);
   const int b1 = s.w[0].sel[0];
-  const uint32_t f = b1 > 0 ? (uint32_t)b1 << 4 : 1u;  // 1: every valid item
+  if (b1 < 0) {
+    res.ok = false;
+    return res;
+  }
+  const uint32_t f = max((uint32_t)b1 << 4, 1u);  // at least k items reach it
 #pragma unroll
   for (int o = 0; o < NO; ++o)
 #pragma unroll
@@ -228,22 +238,14 @@ __device__ __forceinline__ OctResult octn_top(const uint4 (&w)[NO], int k, IdFn 
   fs_rank_bin(hitem, s.w[1], k);
   __syncthreads();
   const int bin = s.w[1].sel[0];
-  uint32_t v = 1;
-  int need = 0, ties = 0;
-  if (bin < 0) {  // fewer than k valid items (f = 1): all of them are members
-    res.sel.all = true;
-    res.sel.above = s.w[1].sel[2];
-  } else {
-    if (bin == 4095) {
-      res.ok = false;
-      return res;
-    }
-    v = f + (uint32_t)bin;
-    res.sel.v = v;
-    res.sel.above = s.w[1].sel[1];
-    need = k - res.sel.above;
-    ties = (int)hitem[bin];
+  if (bin == 4095) {
+    res.ok = false;
+    return res;
   }
+  const uint32_t v = f + (uint32_t)bin;
+  res.sel.v = v;
+  res.sel.above = s.w[1].sel[1];
+  const int need = k - res.sel.above, ties = (int)hitem[bin];
   if (RULE == TIE_VALUE) return res;
   uint32_t gt = 0, eq = 0;
 #pragma unroll
@@ -254,7 +256,7 @@ __device__ __forceinline__ OctResult octn_top(const uint4 (&w)[NO], int k, IdFn 
       gt |= (uint32_t)(x > v) << (8 * o + e);
       eq |= (uint32_t)(x == v) << (8 * o + e);
     }
-  if (need >= ties) {  // (also when all are members)
+  if (need >= ties) {
     res.mine = gt | eq;
     return res;
   }

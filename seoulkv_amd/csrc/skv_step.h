@@ -42,7 +42,8 @@ enum {
   ST_WORDS = 8
 };
 
-// ST_FULLSEL bits: the sampled cut missed and the full selection ran
+// ST_FULLSEL bits: the sampled cut (or, for lists of 8K-32K centroids, the
+// bound of the thread maxima) missed and a selection over every item ran
 enum {
   FS_THRESH = 1,
   FS_FINE = 2,

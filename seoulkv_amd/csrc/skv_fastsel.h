@@ -533,10 +533,14 @@ __device__ __forceinline__ uint32_t tie_cut(int ties, int need, IdFn id, FastScr
 // from its registers (emit(tile, 16-bit mask), once per tile with members).
 // No candidate list is written or read (12.7 -> 10.8 us for the top-1600 of
 // 40K keys).  id(position): an item's ID, read for items tied at the k-th
-// score only.  Returns false, with nothing emitted, when the sample's cut
-// missed (fewer than k items reach it), the k-th score is 4095 or more steps
-// above the cut, or more than FS_TIE_RANK items tie at it: the caller runs
-// another selection.  The scratch is cleared by tiled_clear and a barrier.
+// score only.  A k-th score 4095 or more steps above the cut (scores on both
+// sides of zero) takes two more passes over the registers, and more than
+// FS_TIE_RANK ties at it are cut by a digit count of their IDs, so neither
+// needs another selection (top-1600 of 20K keys, 1650 of them above zero 25.8
+// -> 18.8 us, 2500 of them tied 32.3 -> 20.6 us against selecting again; both
+// branches are marked unlikely: pools without them keep 9.9-10.0 us).  Returns false, with nothing emitted, when the
+// sample's cut missed (fewer than k items reach it): the caller runs another
+// selection.  The scratch is cleared by tiled_clear and a barrier.
 __device__ __forceinline__ void tiled_clear(FastScratch& s) {
   fs_clear(s.hist, s.w[0]);
   fs_clear(s.hist_b, s.w[1]);
@@ -588,13 +592,8 @@ __device__ __forceinline__ bool tiled_select(const TileSrc& src, const uint16_t*
     return oct_at_least(tw[r][0], cm1) | (oct_at_least(tw[r][1], cm1) << 8);
   };
   uint32_t cand[TL_ROUNDS];  // the tiles' items at or above the cut
-#pragma unroll
-  for (int r = 0; r < TL_ROUNDS; ++r) {
-    if (r * SEL_BLOCK >= nhot) break;  // block-uniform
-    uint32_t mask = at_least(r, cut);
-    if (tl[r] < 0) mask = 0;
-    else if (n - 16 * tl[r] < 16) mask &= (1u << (n - 16 * tl[r])) - 1u;
-    cand[r] = mask;
+  // f(score) of the items of round r in mask
+  auto scores_in = [&](int r, uint32_t mask, auto f) {
 #pragma unroll
     for (int q = 0; q < 2; ++q) {  // compile-time octet: no indexed arrays
       uint32_t m8 = (mask >> (8 * q)) & 0xffu;
@@ -602,10 +601,19 @@ __device__ __forceinline__ bool tiled_select(const TileSrc& src, const uint16_t*
         const int e = __ffs(m8) - 1;
         m8 &= m8 - 1;
         const uint32_t word = tw[r][q][e >> 1];
-        const uint32_t o = (e & 1) ? word >> 16 : word & 0xffffu;
-        atomicAdd(&s.hist_b[min(o - cut, 4095u)], 1u);
+        f((e & 1) ? word >> 16 : word & 0xffffu);
       }
     }
+  };
+#pragma unroll
+  for (int r = 0; r < TL_ROUNDS; ++r) {
+    cand[r] = 0;
+    if (r * SEL_BLOCK >= nhot) continue;  // block-uniform
+    uint32_t mask = at_least(r, cut);
+    if (tl[r] < 0) mask = 0;
+    else if (n - 16 * tl[r] < 16) mask &= (1u << (n - 16 * tl[r])) - 1u;
+    cand[r] = mask;
+    scores_in(r, mask, [&](uint32_t o) { atomicAdd(&s.hist_b[min(o - cut, 4095u)], 1u); });
   }
   __syncthreads();
   SKV_TS(ts, 8);
@@ -618,12 +626,34 @@ __device__ __forceinline__ bool tiled_select(const TileSrc& src, const uint16_t*
   int ties = 0;
   if (bin < 0) {
     if (cut > 1) return false;  // the cut missed
-  } else {
-    if (bin == 4095) return false;
+  } else if (__builtin_expect(bin < 4095, 1)) {
     v = cut + (uint32_t)bin;
     need = k - s.w[1].sel[1];
     ties = (int)s.hist_b[bin];
-    if (need < ties && ties > FS_TIE_RANK) return false;
+  } else {  // the k best lie above the last step: 12 bits, then 4 (as octn_select)
+    SelWords& w = s.w[0];
+    fs_clear(s.hist, w);  // last read before the barriers since the cut
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < TL_ROUNDS; ++r)
+      scores_in(r, cand[r], [&](uint32_t o) {
+        if (o - cut >= 4095u) atomicAdd(&s.hist[o >> 4], 1u);
+      });
+    __syncthreads();
+    fs_rank_bin(s.hist, w, k);
+    __syncthreads();
+    const uint32_t b = (uint32_t)w.sel[0];
+    const int acc = w.sel[1];
+#pragma unroll
+    for (int r = 0; r < TL_ROUNDS; ++r)
+      scores_in(r, cand[r], [&](uint32_t o) {
+        if (o - cut >= 4095u && o >> 4 == b) atomicAdd(&w.hist4[o & 15], 1u);
+      });
+    __syncthreads();
+    const DigitRank d = fs_rank_digit(w, k, acc);
+    v = (b << 4) | (uint32_t)d.digit;
+    need = k - d.above;
+    ties = d.ties;
   }
   const bool rank = bin >= 0 && need < ties;  // only some of the ties are members
   uint32_t mem[TL_ROUNDS], eq[TL_ROUNDS];
@@ -641,7 +671,36 @@ __device__ __forceinline__ bool tiled_select(const TileSrc& src, const uint16_t*
       neq += __popc(eq[r]);
     }
   }
-  if (rank) {  // the `need` lowest IDs among the ties win
+  if (__builtin_expect(rank && ties > FS_TIE_RANK, 0)) {
+    // too many to compare: the need-th lowest ID (< 2^20) by its upper 12 and
+    // lower 8 bits, counted from the largest complement
+    SelWords& w = s.w[0];
+    uint32_t found = 0;
+    int left = need;
+#pragma unroll 1
+    for (int low = 0; low < 2; ++low) {
+      __syncthreads();  // (second pass: every thread has read the first's counts)
+      fs_clear(s.hist, w);
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < TL_ROUNDS; ++r)
+        for (uint32_t rest = eq[r]; rest; rest &= rest - 1) {
+          const uint32_t c = 0xfffffu - id(16 * tl[r] + __ffs(rest) - 1);
+          if (!low) atomicAdd(&s.hist[c >> 8], 1u);
+          else if (c >> 8 == found) atomicAdd(&s.hist[c & 255u], 1u);
+        }
+      __syncthreads();
+      fs_rank_bin(s.hist, w, left);
+      __syncthreads();
+      found = (found << 8) | (uint32_t)w.sel[0];
+      left -= w.sel[1];
+    }
+    const uint32_t idcut = 0xfffffu - found;
+#pragma unroll
+    for (int r = 0; r < TL_ROUNDS; ++r)
+      for (uint32_t rest = eq[r]; rest; rest &= rest - 1)
+        if (id(16 * tl[r] + __ffs(rest) - 1) <= idcut) mem[r] |= rest & (0u - rest);
+  } else if (rank) {  // the `need` lowest IDs among the ties win
     const int slot0 = neq ? atomicAdd(&s.w[1].ntie, neq) : 0;
     int slot = slot0;
 #pragma unroll

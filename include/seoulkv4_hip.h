@@ -132,7 +132,10 @@ int skv_enqueue(void *handle);
 
 /* skv_bind_query and skv_enqueue in one call.  The query rides with the first
  * kernel's arguments (no upload of its own) unless a staged append or a
- * captured step needs one; it stays bound for later calls either way.  Under a
+ * captured step needs one; it stays bound for later calls either way.  If the
+ * call fails no query is bound.  No staging slot is taken, so the host is held
+ * back by the HIP runtime alone (about 75 steps ahead of the device, measured
+ * with ROCm 7.2); synchronise to run less far ahead.  Under a
  * caller's stream capture the captured step holds this query: capture
  * skv_enqueue instead to replay with the query bound last. */
 int skv_run(void *handle, const uint16_t *q_bf16);

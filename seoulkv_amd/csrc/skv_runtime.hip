@@ -898,7 +898,7 @@ int skv_bind_query_device(void* handle, const void* q_dev, void* producer_stream
 // One step; query (host memory, or NULL: the bound query in device memory)
 // travels with the front kernel's arguments.
 static int enqueue_step(Handle* h, const QueryArg* query) {
-  if (!h->bound) return fail(h, SKV_ESTATE, "bind a query before enqueue");
+  if (!query && !h->bound) return fail(h, SKV_ESTATE, "bind a query before enqueue");
   HIPCHK(h, hipSetDevice(h->device));
   // a pending host append: packed by this step's k_front (eager launches),
   // or now, before a captured step that takes no append arguments
@@ -960,8 +960,12 @@ int skv_run(void* handle, const uint16_t* q) {
   }
   QueryArg arg;
   memcpy(arg.q, q, sizeof arg.q);
-  h->bound = true;
-  return enqueue_step(h, &arg);
+  // the front kernel stores the query: bound once it is launched, and after a
+  // failure no query is (neither this one nor an older one that a later step
+  // or dense decode would silently use)
+  const int rc = enqueue_step(h, &arg);
+  h->bound = rc == SKV_OK;
+  return rc;
 }
 
 int skv_graph_mode(void* handle, int enable) {

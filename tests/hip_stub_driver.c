@@ -176,9 +176,28 @@ static void output_lifetime(void) {
   CHECK(live == 0, "%d allocations left", live);
 }
 
+/* A run whose launch fails binds nothing: neither its own query, which no
+ * kernel stored, nor the one before it. */
+static void failed_run(void) {
+  void *h = create();
+  CHECK(skv_enqueue(h) == SKV_ESTATE, "enqueue without a query");
+  CHECK(skv_run(h, NULL) == SKV_EINVAL, "NULL query");
+  for (int good = 0; good < 2; ++good) {  /* on the first call, and after a good one */
+    if (good) CHECK(skv_run(h, query) == SKV_OK && skv_enqueue(h) == SKV_OK, "good run");
+    fail_launch = launches;
+    CHECK(skv_run(h, query) == SKV_EHIP, "failing run");
+    CHECK(skv_enqueue(h) == SKV_ESTATE, "enqueue after a failed run");
+    CHECK(skv_dense_decode(h) == SKV_ESTATE, "dense decode after a failed run");
+  }
+  CHECK(skv_bind_query(h, query) == SKV_OK && skv_enqueue(h) == SKV_OK &&
+            skv_dense_decode(h) == SKV_OK, "bound again");
+  skv_destroy(h);
+}
+
 int main(int argc, char **argv) {
   static const struct { const char *name; void (*fn)(void); } scenarios[] = {
       {"output_lifetime", output_lifetime},
+      {"failed_run", failed_run},
   };
   for (size_t i = 0; i < sizeof scenarios / sizeof scenarios[0]; ++i)
     if (argc == 2 && !strcmp(argv[1], scenarios[i].name)) {

@@ -35,7 +35,7 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["output_lifetime"])
+@pytest.mark.parametrize("scenario", ["output_lifetime", "failed_run"])
 def test_host_code_over_the_stub_runtime(driver, scenario):
     res = subprocess.run([str(driver), scenario], capture_output=True, text=True, timeout=120)
     assert res.returncode == 0, (res.returncode, res.stdout, res.stderr)

@@ -6,7 +6,7 @@ them through its page table.  Every result must be bit-identical to the
 contiguous layout's on the same inputs (top-100 IDs, the attention output
 bits, the dense decode's output bits, the records read back in token order),
 the top-100 IDs must equal the oracle's, and the output must stay within the
-north-star bound of the oracle (max-abs <= 2e-2, cosine >= 0.999).  Pages of
+bound of the other parity tests (max-abs <= 2e-2, cosine >= 0.999).  Pages of
 16 tokens put every 16-key tile and every sink/local slice across page
 boundaries; pages of 4096 hold the whole sink and local window in two pages,
 and one page of 65536 tokens holds the whole cache.
@@ -20,7 +20,8 @@ import numpy as np
 import pytest
 import torch
 
-from seoulkv_amd import KVPagePool, SeoulKV4, SeoulKV4Config, _hip
+from seoulkv_amd import KVPagePool, SeoulKV4, SeoulKV4Config, SeoulKV4Index, _hip
+from seoulkv_amd.synthetic import make_cache
 from tests.helpers import bits, case, cosine, oracle_step
 from tests.test_gpu_append import CAPACITY, P, fp8_bytes, new_tokens, oracle_grown
 
@@ -290,3 +291,39 @@ def test_handles_on_concurrent_streams():
     finally:
         for rt in rts:
             rt.close()
+
+
+@pytest.mark.parametrize("page_tokens", [16, 256])
+@pytest.mark.parametrize("context", [24580, 40008])
+def test_paged_dense_decode_past_one_pair_per_wave(context, page_tokens):
+    """Past 12 x 64 pairs of tiles a wave reads its later pairs through the
+    page table as well: some waves with a second pair and others without, and
+    a last pair that ends inside its first tile, inside its second tile (the
+    one moved back while it lies past the context), on a tile and on a pair,
+    as appends move the end.  Bit for bit the contiguous decode, whose edges
+    ``test_gpu_dense_tiles.py`` checks against float64."""
+    capacity = 96
+    k, v, qs = make_cache(context, 512, n_queries=1)
+    index = SeoulKV4Index.build(k, v, nprobe=64, n_centroids=512, build_device="cuda")
+    kw = dict(pool_min=0, pool_capacity=None, debug=False, append_capacity=capacity)
+    need = -(-(context + capacity) // page_tokens)
+    pool = scrambled_pool(need + 5, page_tokens, context)
+    flat = _hip.Runtime(0, k, v, index, **kw)
+    paged = _hip.Runtime(0, k, v, index, kv_pages=(pool, pool.allocate(need)), **kw)
+    gen = torch.Generator().manual_seed(context)
+    try:
+        for rt in (flat, paged):
+            rt.bind_query(qs[0])
+        for end in (context % 32, 15, 16, 17, 31, 0, 1):  # T modulo a pair
+            n = (end - flat.T) % 32
+            if n:
+                kn, vn = (torch.randn(4, n, 256, generator=gen).bfloat16() for _ in range(2))
+                flat.append(kn, vn)
+                paged.append(kn, vn)
+            print(f"[gpu] paged dense T={flat.T} pages of {page_tokens}", flush=True)
+            out = dense(flat)
+            assert torch.equal(dense(paged), out), flat.T
+            assert torch.isfinite(out.view(torch.bfloat16)).all()
+    finally:
+        paged.close()
+        flat.close()

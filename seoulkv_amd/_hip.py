@@ -499,6 +499,7 @@ class Runtime:
         if getattr(self, "handle", None):
             self.lib.skv_destroy(self.handle)
             self.handle = None
+        self._pool = None  # no handle reads the pages any more
 
     def __del__(self):
         try:

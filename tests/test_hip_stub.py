@@ -66,9 +66,14 @@ class _Lib:
         return 0
 
 
+class _Pages:
+    """Stands for a page pool, whose device memory goes with the object."""
+
+
 def _instance(lib):
     runtime = _hip.Runtime.__new__(_hip.Runtime)
     runtime.lib, runtime.handle, runtime.device = lib, 0x55, 0
+    runtime._pool = _Pages()
     runtime.output = _hip.OutputMemory(lib, runtime.handle)
     attn = SeoulKV4.__new__(SeoulKV4)
     attn._state, attn._closed, attn._generation, attn._device = runtime, False, 1, 0
@@ -97,12 +102,14 @@ def views(monkeypatch):
 def test_output_view_keeps_the_outputs_and_nothing_else(views, how):
     lib = _Lib()
     attn = _instance(lib)
+    pages = weakref.ref(attn._state._pool)
     view = DecodeResult(attn, 1).device_tensors
     if how == "close":
         attn.close()
     del attn
     gc.collect()
     assert lib.events == ["caches"]  # freed under the live view, the outputs not
+    assert pages() is None
     del view
     gc.collect()
     assert lib.events == ["caches", "outputs"]

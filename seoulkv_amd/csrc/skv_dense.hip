@@ -195,11 +195,13 @@ __device__ __forceinline__ int fp8_bf16x2(uint32_t w) {
 // registers and widened to BF16 (exact), are its row operand, and the
 // column operand of lane (kb, 4h + s) is made from the scores that the lane
 // itself holds (head h, the same 8 keys): no value moves between lanes.  A
-// probability enters exactly, as three BF16 terms (8 + 8 + 8 significant
-// bits) in the columns s = 0, 1, 2 (s = 3: zero); the epilogue adds the
-// columns.  The products are exact and summed in FP32.  m is the running
-// max of head h over all the wave's keys (it moves by more than DN_TAU or
-// not at all), l the sum over this lane's keys.
+// probability enters as three BF16 terms (8 + 8 + 8 significant bits) in the
+// columns s = 0, 1, 2 (s = 3: zero), exactly down to 2^-110, where the third
+// term's last bit reaches BF16's smallest step (2^-133); the epilogue adds the
+// columns.  (exp2 is the bare instruction: a p below 2^-126 is 0.)  The
+// products are exact and summed in FP32.  m is the running max of head h over
+// all the wave's keys (it moves by more than DN_TAU or not at all), l the sum
+// over this lane's keys.
 template <bool TAIL, typename NextK>
 __device__ __forceinline__ void dn_pair(DnPair& x, int t0, int T, int lane, const DenseImage& img,
                                         float zc, v4f (&o)[16], float& m, float& l, NextK next_k) {
@@ -314,8 +316,8 @@ __device__ __forceinline__ float2* dense_stats(float* part, int nb) {
 // three pairs in 4 waves of 512, spilled.)  Whole call with the merge, back
 // to back, against V sums on the vector ALUs (half of every SIMD's cycles)
 // with the query formed by every wave: T = 1000 16.6 -> 8.5 us, 40009 27 ->
-// 21, 131072 54.8 -> 47.1, 2^20 374 -> 310 (6.9 TB/s); the reload below took
-// the middle two to 18 and 43-45 later.
+// 18, 131072 51-55 -> 45-47 (43 without the merge), 2^20 374 -> 310
+// (6.9 TB/s), with the reload below.
 // The arguments are DenseArgs' fields as scalars, preloaded at dispatch: the
 // first loads need not wait for an argument block.
 template <bool PAGED>

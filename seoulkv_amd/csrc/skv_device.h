@@ -118,40 +118,6 @@ __host__ __device__ inline float sqrt_rne_scaled(unsigned long long N, int fx) {
   return (float)ldexp((double)qv, drop - k + fx);
 }
 
-// FP8 e4m3fn (OCP: bias 7, no infinities, S.1111.111 = NaN) -> FP32, exact.
-__host__ __device__ inline float fp8_e4m3_to_f32(uint32_t b) {
-  const uint32_t sign = (b & 0x80u) << 24;
-  const uint32_t e = (b >> 3) & 15u, m = b & 7u;
-  if (e == 0) {
-    const float v = (float)m * 0.001953125f;  // m * 2^-9
-    return sign ? -v : v;
-  }
-  if (e == 15 && m == 7) return u2f(0x7fc00000u | sign);
-  return u2f(sign | ((e + 120u) << 23) | (m << 20));
-}
-
-// FP32 -> FP8 e4m3fn, round to nearest even; magnitudes above 464 (the
-// midpoint past 448) and NaN/Inf become NaN (0x7f | sign), as torch's
-// float8_e4m3fn cast does.
-__host__ __device__ inline uint32_t f32_to_fp8_e4m3(float f) {
-  uint32_t u = f2u(f);
-  const uint32_t sign = (u >> 24) & 0x80u;
-  u &= 0x7fffffffu;
-  if (u > 0x7f800000u || u == 0x7f800000u) return sign | 0x7fu;
-  if (u < 0x3c800000u) {  // below 2^-6: subnormal grid of 2^-9
-    const float scaled = u2f(u) * 512.0f;  // exact
-    uint32_t m = (uint32_t)scaled;
-    const float frac = scaled - (float)m;
-    if (frac > 0.5f || (frac == 0.5f && (m & 1u))) ++m;
-    return sign | m;  // m == 8 is the smallest normal (0x08)
-  }
-  const uint32_t r = u + 0x7ffffu + ((u >> 20) & 1u);
-  const int e = (int)(r >> 23) - 127 + 7;
-  const uint32_t m = (r >> 20) & 7u;
-  if (e > 15 || (e == 15 && m == 7)) return sign | 0x7fu;
-  return sign | ((uint32_t)e << 3) | m;
-}
-
 // Four BF16 values (packed in w) -> four FP8 e4m3fn bytes (torch's cast).
 // The gfx950 converter (v_cvt_pk_fp8_f32, round to nearest even) gives
 // torch's byte for every finite and infinite BF16 input (checked on all
@@ -195,20 +161,6 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 __device__ __forceinline__ int wave_sum(int v) {
   return __builtin_amdgcn_readlane(wave_incl_scan(v), 63);
 }
-
-// Float wave total (tree order fixed by the DPP pattern), uniform across lanes.
-#define SKV_DPP_ADDF(v, ctrl, rows, zero) \
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, zero))
-__device__ __forceinline__ float wave_sum_f(float v) {
-  SKV_DPP_ADDF(v, 0x111, 0xf, true);   // row_shr:1
-  SKV_DPP_ADDF(v, 0x112, 0xf, true);   // row_shr:2
-  SKV_DPP_ADDF(v, 0x114, 0xf, true);   // row_shr:4
-  SKV_DPP_ADDF(v, 0x118, 0xf, true);   // row_shr:8
-  SKV_DPP_ADDF(v, 0x142, 0xa, false);  // row_bcast:15
-  SKV_DPP_ADDF(v, 0x143, 0xc, false);  // row_bcast:31
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-#undef SKV_DPP_ADDF
 
 __device__ __forceinline__ int wave_max(int v) {
   constexpr int LO = (int)0x80000000;

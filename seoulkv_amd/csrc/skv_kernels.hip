@@ -601,8 +601,9 @@ __global__ __launch_bounds__(FR_BLOCK) void k_front(const uint16_t* __restrict__
 
 // The front of a step whose query was bound from host memory since the last
 // one: the 8 KiB query comes as a kernel argument, so the step needs no
-// upload of its own (an in-stream copy before the front kernel cost 3.6 us of
-// every step: 128K 55.5 -> 52.7 us, 8K 44 -> 41, a new query per step).
+// upload of its own (an in-stream copy before the front kernel cost about 3 us
+// of every step: bench.py's host loop at 128K 54.4 us with bind + enqueue, 51.4
+// with run).
 template <bool LOOP>
 __global__ __launch_bounds__(FR_BLOCK) void k_front_bind(StepArgs a, QueryArg qa) {
   front_body<LOOP, false, true>(qa.q, a);

@@ -60,10 +60,9 @@ enum TieRule {
 // barrier of the caller's before they, or s.tie, are used again.
 //
 // These selections run on one CU with 16 waves, so their time is the number
-// of block-wide phases: five barriers (counts, two for the bin, digit, ties)
-// against 13 when the caller's scratch was cleared inside, one wave worked
-// out each rank for the others, and the tied items went through a position
-// list (top-256 of 6000 keys 5.4 -> 4.6 us, threshold and fine selection of
+// of block-wide phases: six barriers (cleared scratch, counts, two for the
+// bin, digit, ties) against 13 when one wave worked out each rank for the
+// others and the tied items went through a position list (top-256 of 6000 keys 5.4 -> 4.6 us, threshold and fine selection of
 // 8192 centroids 5.9 -> 4.9 us).
 template <int NO, TieRule RULE, typename IdFn>
 __device__ __forceinline__ OctResult octn_select(const uint4 (&w)[NO], int k, IdFn id,

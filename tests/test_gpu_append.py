@@ -2,7 +2,7 @@
 
 After n appended tokens the step must equal the oracle's step over the grown
 cache (context T0 + n, local window L + n, the prefill's index, codes and
-scales): top-100 IDs bit for bit, the attention output within the north-star
+scales): top-100 IDs bit for bit, the attention output within the parity
 bound (max-abs <= 2e-2, cosine >= 0.999 per query head).  The appended FP8
 records must equal torch's FP8 e4m3fn cast of the BF16 inputs bit for bit.
 The appended keys lean towards the query, so the output moves visibly when

@@ -1,7 +1,7 @@
 """Dense FP8 decode (the comparison path) against the oracle's float64
 softmax over all T keys of the same FP8 [V || K] records.
 
-Tolerance: the north-star bound (max-abs <= 2e-2, cosine >= 0.999 per query
+Tolerance: the parity bound (max-abs <= 2e-2, cosine >= 0.999 per query
 head) and, tighter, |out - ref| <= 2^-8 |ref| + 1e-4: the output is BF16 (RNE,
 half an ulp <= 2^-8 relative) of an FP32 result, so a dropped query term
 (2^-4 relative), a lost key or a wrong softmax scale fails it.

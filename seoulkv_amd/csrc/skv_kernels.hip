@@ -694,8 +694,9 @@ __device__ __forceinline__ void select_in_registers_n(const StepArgs& a, const u
   uint32_t missed = 0;  // ST_FULLSEL bits
   OctResult r1;
   r1.ok = false;
-  if (P <= SEL_BLOCK) r1 = octn_top<NO, TIE_VALUE>(wl, P, cid, fs.hist, fs.hist_b, fs, 2);
-  if (!r1.ok) {
+  if (__builtin_expect(P <= SEL_BLOCK, 1))
+    r1 = octn_top<NO, TIE_VALUE>(wl, P, cid, fs.hist, fs.hist_b, fs, 2);
+  if (__builtin_expect(!r1.ok, 0)) {
     missed |= FS_THRESH;
     __syncthreads();
     fs_clear(fs.hist, fs.w[0]);
@@ -715,16 +716,18 @@ __device__ __forceinline__ void select_in_registers_n(const StepArgs& a, const u
   OctResult r2;
   r2.ok = false;
   r2.sel.v = 0;
-  if (P <= SEL_BLOCK) r2 = octn_top<NO, TIE_ID>(wm, P, cid, fs.hist_c, fs.hist, fs, 4);
-  if (!r2.ok) missed |= FS_FINE;
-  if (!r2.ok && r2.sel.v == 0) {
+  if (__builtin_expect(P <= SEL_BLOCK, 1))
+    r2 = octn_top<NO, TIE_ID>(wm, P, cid, fs.hist_c, fs.hist, fs, 4);
+  if (__builtin_expect(!r2.ok, 0)) missed |= FS_FINE;
+  if (__builtin_expect(!r2.ok && r2.sel.v == 0, 0)) {
     __syncthreads();
     fs_clear(fs.hist, fs.w[0]);
     __syncthreads();
     r2 = octn_select<NO, TIE_ID>(wm, P, cid, fs.hist, fs.w[0], fs, 4);
   }
-  if (missed && t == 0) atomicOr(&a.status[g * ST_WORDS + ST_FULLSEL], missed);
-  if (r2.ok) {
+  if (__builtin_expect(missed, 0) && t == 0)
+    atomicOr(&a.status[g * ST_WORDS + ST_FULLSEL], missed);
+  if (__builtin_expect(r2.ok, 1)) {
     // items 8u .. 8u+7 (u = t + o SEL_BLOCK) are byte u & 3 of bitmap word u >> 2
 #pragma unroll
     for (int o = 0; o < NO; ++o) {
@@ -1918,6 +1921,40 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
   SKV_TS(13, 15);
   SKV_TSE(9);
 }
+
+// The instances in the order in which their code lies: those of a default step
+// together, the long-list selections (28-39 KB each) last.  The seven kernels
+// run about 60 KB of instructions between them, close to what an instruction
+// cache holds, and a step's time moves with their places: of seven orders of
+// the same code, 128K steps took 51.3-52.0 us with contiguous and 51.4-52.6
+// with paged records; left to the order of use, code added to the long-list
+// selections made one of the two 0.5 us slower.  This one: 51.5 and 52.05.
+template __global__ void k_topk<false>(const int*, const uint16_t*, int, int, const uint16_t*, int,
+                                       TopkArgs);
+template __global__ void k_top100<false>(const int*, const uint16_t*, const int*, const uint64_t*, int,
+                                         const uint16_t*, const float*, int, int, StepArgs);
+template __global__ void k_top100<true>(const int*, const uint16_t*, const int*, const uint64_t*, int,
+                                         const uint16_t*, const float*, int, int, StepArgs);
+template __global__ void k_select<false, 1>(const uint16_t*, const uint16_t*, const uint16_t*, int, int,
+                                         int, StepArgs);
+template __global__ void k_select<true, 1>(const uint16_t*, const uint16_t*, const uint16_t*, int, int,
+                                         int, StepArgs);
+template __global__ void k_front_bind<false>(StepArgs, QueryArg);
+template __global__ void k_front<false, false>(const uint16_t* __restrict__, StepArgs);
+template __global__ void k_front_bind<true>(StepArgs, QueryArg);
+template __global__ void k_front<true, false>(const uint16_t* __restrict__, StepArgs);
+template __global__ void k_front<false, true>(const uint16_t* __restrict__, StepArgs);
+template __global__ void k_front<true, true>(const uint16_t* __restrict__, StepArgs);
+template __global__ void k_topk<true>(const int*, const uint16_t*, int, int, const uint16_t*, int,
+                                       TopkArgs);
+template __global__ void k_select<false, 2>(const uint16_t*, const uint16_t*, const uint16_t*, int, int,
+                                         int, StepArgs);
+template __global__ void k_select<true, 2>(const uint16_t*, const uint16_t*, const uint16_t*, int, int,
+                                         int, StepArgs);
+template __global__ void k_select<false, 4>(const uint16_t*, const uint16_t*, const uint16_t*, int, int,
+                                         int, StepArgs);
+template __global__ void k_select<true, 4>(const uint16_t*, const uint16_t*, const uint16_t*, int, int,
+                                         int, StepArgs);
 
 // ============================================================ launcher
 const char* const kKernelNames[N_STEP_KERNELS] = {

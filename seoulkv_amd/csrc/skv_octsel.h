@@ -220,7 +220,7 @@ __device__ __forceinline__ OctResult octn_top(const uint4 (&w)[NO], int k, IdFn 
   __syncthreads();
   SKV_TS(ts, 2);
   const int b1 = s.w[0].sel[0];
-  if (b1 < 0) {
+  if (__builtin_expect(b1 < 0, 0)) {
     res.ok = false;
     return res;
   }
@@ -237,7 +237,7 @@ __device__ __forceinline__ OctResult octn_top(const uint4 (&w)[NO], int k, IdFn 
   fs_rank_bin(hitem, s.w[1], k);
   __syncthreads();
   const int bin = s.w[1].sel[0];
-  if (bin == 4095) {
+  if (__builtin_expect(bin == 4095, 0)) {
     res.ok = false;
     return res;
   }
@@ -259,7 +259,7 @@ __device__ __forceinline__ OctResult octn_top(const uint4 (&w)[NO], int k, IdFn 
     res.mine = gt | eq;
     return res;
   }
-  if (ties > FS_TIE_RANK) {
+  if (__builtin_expect(ties > FS_TIE_RANK, 0)) {
     res.ok = false;
     return res;
   }

@@ -1923,12 +1923,12 @@ __global__ __launch_bounds__(SEL_BLOCK) void k_top100(const int* status, const u
 }
 
 // The instances in the order in which their code lies: those of a default step
-// together, the long-list selections (28-39 KB each) last.  The seven kernels
-// run about 60 KB of instructions between them, close to what an instruction
-// cache holds, and a step's time moves with their places: of seven orders of
-// the same code, 128K steps took 51.3-52.0 us with contiguous and 51.4-52.6
-// with paged records; left to the order of use, code added to the long-list
-// selections made one of the two 0.5 us slower.  This one: 51.5 and 52.05.
+// together, the long-list selections (28-39 KB each) last.  A step's time
+// moves with the places of its kernels' code, for a reason not found (aligning
+// each to 4 or 8 KiB changes nothing): in different orders of the same code
+// 128K steps took 51.3-52.0 us with contiguous and 51.4-52.6 with paged
+// records, and left to the order of use, code added to the long-list
+// selections made one of the two 0.5 us slower.  This order: 51.4 and 52.0.
 template __global__ void k_topk<false>(const int*, const uint16_t*, int, int, const uint16_t*, int,
                                        TopkArgs);
 template __global__ void k_top100<false>(const int*, const uint16_t*, const int*, const uint64_t*, int,

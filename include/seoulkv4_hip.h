@@ -161,8 +161,8 @@ int skv_output_tiles_device(void *handle, void **dev_ptr);
  * skv_dense_output_device: it stays allocated (about 0.3 MiB, with the last
  * values written) until the hold is released, also past skv_destroy, which
  * frees everything else.  Each hold is released once, from any thread, after
- * the work that reads the outputs has been enqueued.  The reference leaves
- * views of a closed instance to TT-NN's own reference counts. */
+ * the work that reads the outputs has been enqueued.  (No counterpart in the
+ * reference.) */
 int skv_output_hold(void *handle, void **hold);
 void skv_output_release(void *hold);
 
